@@ -346,42 +346,87 @@ __device__ __forceinline__ void utab(const Geo &g, int f, R T[GK_RECW_STRIDE]) {
   for (int n = 0; n < GK_RECW_STRIDE; n++) T[n] = c[n];
 }
 
+// PDMU7 limiter (reference src/solver_func.c:215-253) of both states of a
+// face.  The reference limits one state from the unlimited interpolant f_itp
+// and three cells of the upwind frame, f-1, f0 and f+1 (the last two are the
+// face's own cells, in either order):
+//   f    = max(min(f0, f+1), min(f_itp, max(f0, f+1)))
+//   df0c = 0.5 |f0 - f-1| + 0.25 |c1 f0 + c2 f-1|
+//   out  = f - s1 max(0, |f - f0| - |s0 + s1| df0c),  s0, s1 the signs of
+//          f0 - f-1 and f+1 - f0
+// with the geometry terms c1, c2 precomputed per face.  Everything that is a
+// power of two is folded here, which changes no rounding (underflow aside):
+// |s0 + s1| df0c is q D with D = |f0 - f-1| + 0.5 |c1 f0 + c2 f-1| and q = 1,
+// 0.5, 0 for equal signs, f0 = f-1, opposite signs, and q D is exact inside a
+// fused multiply-add.  s1 multiplies a number that is 0 where s1 is 0
+// (f0 = f+1 clamps f to f0), so it is a copied sign bit; the other state of
+// the face has the opposite s1.  The signs are read off the high words
+// instead of being formed as -1, 0, 1 (two compares and a select or two
+// each).  The sweeps and edge fields are bound by vector issue (72-92 % busy
+// in the sweeps), and this is 22 vector instructions per state in FP64
+// against 33: 256^3 FP64 i / j / k sweeps 1.06 / 1.04 / 1.22 -> 0.97 / 0.97 /
+// 1.17 ms, E_i / E_j / E_k 0.351 / 0.387 / 0.520 -> 0.331 / 0.372 / 0.507 ms,
+// FP32-bulk sweeps 0.46 -> 0.44 ms (there memory binds next).
+__device__ __forceinline__ double limit_q(double d0, double d1) {
+  const int differ = __double2hiint(d0) ^ __double2hiint(d1);
+  int hi = differ < 0 ? 0 : 0x3FF00000;  // 0, 1
+  hi = d0 == 0.0 ? 0x3FE00000 : hi;      // 0.5
+  return __hiloint2double(hi, 0);
+}
+__device__ __forceinline__ float limit_q(float d0, float d1) {
+  const float q = (__float_as_int(d0) ^ __float_as_int(d1)) < 0 ? 0.0f : 1.0f;
+  return d0 == 0.0f ? 0.5f : q;
+}
+__device__ __forceinline__ double with_sign(double a, double s) { return __builtin_copysign(a, s); }
+__device__ __forceinline__ float with_sign(float a, float s) { return __builtin_copysignf(a, s); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// The excess max(0, |f - f0| - q D) that the limiter takes off a state
 template <typename R>
-__device__ __forceinline__ R sgn(R x) {
-  return (x > R(0)) ? R(1) : ((x < R(0)) ? R(-1) : R(0));
+__device__ __forceinline__ R pdm_excess(R f, R fm1, R f0, R d0, R d1, R c1, R c2) {
+  const R g = madd(c2, fm1, c1 * f0);
+  const R D = fma_r(R(0.5), fabs(g), fabs(d0));
+  return fmax(R(0), fma_r(-limit_q(d0, d1), D, fabs(f - f0)));
 }
 
-// PDMU7 limiter (reference src/solver_func.c:215-253) given the unlimited
-// interpolant and the three limiter cells (i-1, i, i+1 in the upwind frame);
-// the geometry ratio terms (q - e A_i)/(e A_i) and (e A_im1 - q)/(e A_i) are
-// precomputed per face as c1, c2 (the reference forms them first as well).
+// Limited left and right states of a face from the unlimited interpolants and
+// the cells f-2 .. f+1 around it; T: the face's table
 template <typename R>
-__device__ __forceinline__ R pdm_limit(R f_itp, R fm1, R f0, R fp1, R c1, R c2) {
-  R maxf = fmax(f0, fp1), minf = fmin(f0, fp1);
-  R f = fmax(minf, fmin(f_itp, maxf));
-  R df0 = f0 - fm1, df1 = fp1 - f0;
-  R s0 = sgn(df0), s1 = sgn(df1);
-  df0 = fabs(df0);
-  R q0 = fabs(s0 + s1);
-  R dfl = f - f0;
-  R df0c = fabs(madd(c2, fm1, c1 * f0)) / R(2);
-  df0c = madd(R(0.5), df0, R(0.5) * df0c);
-  // f - s1 max(0, |dfl| - q0 df0c), with x - y z written x + (-y) z
-  return madd(-s1, fmax(R(0), madd(-q0, df0c, fabs(dfl))), f);
+__device__ __forceinline__ void pdm_pair(R fl, R fr, R xm2, R xm1, R x0, R xp1, const R *T, R &L,
+                                         R &Rr) {
+  const R maxf = fmax(xm1, x0), minf = fmin(xm1, x0);
+  const R d = x0 - xm1;
+  fl = fmax(minf, fmin(fl, maxf));
+  fr = fmax(minf, fmin(fr, maxf));
+  const R tl = pdm_excess(fl, xm2, xm1, xm1 - xm2, d, T[14], T[15]);
+  // seen from the right state the differences are x0 - xp1 and -d: both negated
+  const R tr = pdm_excess(fr, xp1, x0, xp1 - x0, d, T[16], T[17]);
+  L = fl - with_sign(tl, d);
+  Rr = fr + with_sign(tr, d);
+}
+
+// Unlimited interpolants of a face from the half-step values of its 8 cells.
+// Each sum starts with its first product (the reference adds it to 0, which
+// only turns a -0 into +0).
+template <typename R>
+__device__ __forceinline__ void interpolate(const R xh[8], const R *T, R &fl, R &fr) {
+  fl = xh[0] * T[0];
+  fr = xh[7] * T[7];
+#pragma unroll
+  for (int n = 1; n < 7; n++) {
+    fl = madd(xh[n], T[n], fl);
+    fr = madd(xh[7 - n], T[7 + n], fr);
+  }
 }
 
 // Left/right states at a face from 8 stencil cells (f-4 .. f+3): xh are the
 // half-step values that are interpolated, xn the values that limit.
 template <typename R>
 __device__ __forceinline__ void pdm_lr(const R xh[8], const R xn[8], const R *T, R &L, R &Rr) {
-  R fl = R(0), fr = R(0);
-#pragma unroll
-  for (int n = 0; n < 7; n++) {
-    fl = madd(xh[n], T[n], fl);
-    fr = madd(xh[7 - n], T[7 + n], fr);
-  }
-  L = pdm_limit(fl, xn[2], xn[3], xn[4], T[14], T[15]);
-  Rr = pdm_limit(fr, xn[5], xn[4], xn[3], T[16], T[17]);
+  R fl, fr;
+  interpolate(xh, T, fl, fr);
+  pdm_pair(fl, fr, xn[2], xn[3], xn[4], xn[5], T, L, Rr);
 }
 
 // Reconstruct a stored field p (history q; self-limited when q == nullptr)
@@ -912,15 +957,10 @@ __device__ __forceinline__ void march_shift(Window<NF, R> &w) {
 
 template <int NF, typename R>
 __device__ __forceinline__ void march_lr(const Window<NF, R> &w, int m, const R *T, R &L, R &Rr) {
-  R fl = R(0), fr = R(0);
-#pragma unroll
-  for (int n = 0; n < 7; n++) {
-    fl = madd(w.h[m][n], T[n], fl);
-    fr = madd(w.h[m][7 - n], T[7 + n], fr);
-  }
+  R fl, fr;
+  interpolate(w.h[m], T, fl, fr);
   // limiter cells: x[0] = f-2, x[1] = f-1, x[2] = f, x[3] = f+1
-  L = pdm_limit(fl, w.x[m][0], w.x[m][1], w.x[m][2], T[14], T[15]);
-  Rr = pdm_limit(fr, w.x[m][3], w.x[m][2], w.x[m][1], T[16], T[17]);
+  pdm_pair(fl, fr, w.x[m][0], w.x[m][1], w.x[m][2], w.x[m][3], T, L, Rr);
 }
 
 template <int D, typename R, bool B0V, bool UT>
@@ -1149,14 +1189,9 @@ __device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, 
   const long c = rowb + k;
   const int b = tx;  // stencil cells b .. b+7 in LDS
   auto lr = [&](int m, R &L, R &Rr) {
-    R fl = R(0), fr = R(0);
-#pragma unroll
-    for (int n = 0; n < 7; n++) {
-      fl = madd(sh[m][b + n], T[n], fl);
-      fr = madd(sh[m][b + 7 - n], T[7 + n], fr);
-    }
-    L = pdm_limit(fl, sx[m][b + 2], sx[m][b + 3], sx[m][b + 4], T[14], T[15]);
-    Rr = pdm_limit(fr, sx[m][b + 5], sx[m][b + 4], sx[m][b + 3], T[16], T[17]);
+    R fl, fr;
+    interpolate(&sh[m][b], T, fl, fr);
+    pdm_pair(fl, fr, sx[m][b + 2], sx[m][b + 3], sx[m][b + 4], sx[m][b + 5], T, L, Rr);
   };
   if (!full) {
     R l, rr;
@@ -1300,14 +1335,7 @@ struct Window1 {  // self-limited field: half-step = current value
 
 template <typename R>
 __device__ __forceinline__ void lr_self(const Window1<R> &w, const R *T, R &L, R &Rr) {
-  R fl = R(0), fr = R(0);
-#pragma unroll
-  for (int n = 0; n < 7; n++) {
-    fl = madd(w.h[n], T[n], fl);
-    fr = madd(w.h[7 - n], T[7 + n], fr);
-  }
-  L = pdm_limit(fl, w.h[2], w.h[3], w.h[4], T[14], T[15]);
-  Rr = pdm_limit(fr, w.h[5], w.h[4], w.h[3], T[16], T[17]);
+  pdm_lr(w.h, w.h, T, L, Rr);
 }
 
 template <typename R>
@@ -1361,10 +1389,13 @@ struct TableWalk {
 // per SIMD they have the registers to issue a position's table and field
 // loads together (at three the compiler loads the table piecewise), and at
 // least two keep the compiler from spending more registers than two waves
-// leave (with uniform tables it would otherwise drop to one).
+// leave (with uniform tables it would otherwise drop to one).  The FP64 E_i
+// march with per-lane tables is the same case (96x72x60: 0.042 ms at three
+// waves, 0.032 at two); with uniform tables it holds its direct table across
+// the march and runs best unbounded.
 template <int D, typename R, bool UT>
 struct EmfWaves {
-  static constexpr bool two = sizeof(R) == 8 && D != 0;
+  static constexpr bool two = sizeof(R) == 8 && (D != 0 || !UT);
   static constexpr int lo = two ? 2 : 1;
   static constexpr int hi = two ? 2 : 8;
 };
