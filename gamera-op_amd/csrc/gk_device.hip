@@ -354,15 +354,14 @@ __device__ __forceinline__ void utab(const Geo &g, int f, R T[GK_RECW_STRIDE]) {
 //   df0c = 0.5 |f0 - f-1| + 0.25 |c1 f0 + c2 f-1|
 //   out  = f - s1 max(0, |f - f0| - |s0 + s1| df0c),  s0, s1 the signs of
 //          f0 - f-1 and f+1 - f0
-// with the geometry terms c1, c2 precomputed per face.  Everything that is a
-// power of two is folded here, which changes no rounding (underflow aside):
-// |s0 + s1| df0c is q D with D = |f0 - f-1| + 0.5 |c1 f0 + c2 f-1| and q = 1,
-// 0.5, 0 for equal signs, f0 = f-1, opposite signs, and q D is exact inside a
-// fused multiply-add.  s1 multiplies a number that is 0 where s1 is 0
-// (f0 = f+1 clamps f to f0), so it is a copied sign bit; the other state of
-// the face has the opposite s1.  The signs are read off the high words
-// instead of being formed as -1, 0, 1 (two compares and a select or two
-// each).  The sweeps and edge fields are bound by vector issue (72-92 % busy
+// with the geometry terms c1, c2 precomputed per face.  |s0 + s1| is 2, 1, 0
+// for equal signs, f0 = f-1, opposite signs, so its product is exact inside a
+// fused multiply-add.  In FP64 the halves are folded too (D = 2 df0c, half the
+// factor), which changes no rounding above 1e-307.  s1 multiplies a number
+// that is 0 where s1 is 0 (f0 = f+1 clamps f to f0), so it is a copied sign
+// bit; the other state of the face has the opposite s1.  The signs are read
+// off the high words instead of being formed as -1, 0, 1 (two compares and a
+// select or two each).  The sweeps and edge fields are bound by vector issue (72-92 % busy
 // in the sweeps), and this is 22 vector instructions per state in FP64
 // against 33: 256^3 FP64 i / j / k sweeps 1.06 / 1.04 / 1.22 -> 0.97 / 0.97 /
 // 1.17 ms, E_i / E_j / E_k 0.351 / 0.387 / 0.520 -> 0.331 / 0.372 / 0.507 ms,
@@ -374,20 +373,27 @@ __device__ __forceinline__ double limit_q(double d0, double d1) {
   return __hiloint2double(hi, 0);
 }
 __device__ __forceinline__ float limit_q(float d0, float d1) {
-  const float q = (__float_as_int(d0) ^ __float_as_int(d1)) < 0 ? 0.0f : 1.0f;
-  return d0 == 0.0f ? 0.5f : q;
+  const float q = (__float_as_int(d0) ^ __float_as_int(d1)) < 0 ? 0.0f : 2.0f;
+  return d0 == 0.0f ? 1.0f : q;
 }
 __device__ __forceinline__ double with_sign(double a, double s) { return __builtin_copysign(a, s); }
 __device__ __forceinline__ float with_sign(float a, float s) { return __builtin_copysignf(a, s); }
-__device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-// The excess max(0, |f - f0| - q D) that the limiter takes off a state
-template <typename R>
-__device__ __forceinline__ R pdm_excess(R f, R fm1, R f0, R d0, R d1, R c1, R c2) {
-  const R g = madd(c2, fm1, c1 * f0);
-  const R D = fma_r(R(0.5), fabs(g), fabs(d0));
-  return fmax(R(0), fma_r(-limit_q(d0, d1), D, fabs(f - f0)));
+// The excess max(0, |f - f0| - q D) that the limiter takes off a state.  FP32
+// values do reach the subnormal range, where halving rounds (velocities far
+// from a blob: a last bit of 1e-45 there grows into 1e-6 within 200 steps), so
+// the FP32-bulk form takes its halves one by one as the reference does.
+__device__ __forceinline__ double pdm_excess(double f, double fm1, double f0, double d0, double d1,
+                                             double c1, double c2) {
+  const double g = c1 * f0 + c2 * fm1;
+  const double D = __builtin_fma(0.5, fabs(g), fabs(d0));
+  return fmax(0.0, __builtin_fma(-limit_q(d0, d1), D, fabs(f - f0)));
+}
+__device__ __forceinline__ float pdm_excess(float f, float fm1, float f0, float d0, float d1,
+                                            float c1, float c2) {
+  const float g = madd(c2, fm1, c1 * f0);
+  const float D = madd(0.5f, fabsf(d0), 0.5f * (fabsf(g) * 0.5f));
+  return fmaxf(0.0f, madd(-limit_q(d0, d1), D, fabsf(f - f0)));
 }
 
 // Limited left and right states of a face from the unlimited interpolants and
