@@ -37,6 +37,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -145,19 +146,45 @@ constexpr unsigned long long DBL_INF_BITS = 0x7FF0000000000000ULL;
 // would pause.
 struct Scal {
   double dt, dt0, time, c;
-  unsigned long long smin[NSLOT];  // bit images of partial minima of the next CFL dt (>= 0)
-  unsigned long long smax[NSLOT];  // bit images of partial maxima of |div B|
   unsigned int nanflag;
   unsigned int halt;     // this step's kernels do nothing
   unsigned int stop;     // the next step halts
+  unsigned int ent;      // this step carries the entropy channel (carries_entropy)
+  unsigned int ent_next; // the next steps have to
   unsigned int pad;
   long long budget;      // steps the grid may still take (< 0: no limit)
   long long steps;       // steps taken since the grid was armed
   double t_stop, t_event;
+  double pad2[5];        // the slots, which every block of a launch updates, in lines of their own
+  unsigned long long smin[NSLOT];  // bit images of partial minima of the next CFL dt (>= 0)
+  unsigned long long smax[NSLOT];  // bit images of partial maxima of |div B|
 };
+// 8-byte words of the scalars that k_begin reads
+enum { SW_DT0 = 1, SW_TIME = 2, SW_HALT = 4, SW_STOP = 5, SW_ENT_NEXT = 6, SW_BUDGET = 7,
+       SW_STEPS = 8, SW_T_STOP = 9, SW_T_EVENT = 10, SW_COUNT = 11 };
+static_assert(offsetof(Scal, dt0) == 8 * SW_DT0 && offsetof(Scal, time) == 8 * SW_TIME &&
+                  offsetof(Scal, halt) == 8 * SW_HALT + 4 && offsetof(Scal, stop) == 8 * SW_STOP &&
+                  offsetof(Scal, ent_next) == 8 * SW_ENT_NEXT &&
+                  offsetof(Scal, budget) == 8 * SW_BUDGET && offsetof(Scal, steps) == 8 * SW_STEPS &&
+                  offsetof(Scal, t_stop) == 8 * SW_T_STOP &&
+                  offsetof(Scal, t_event) == 8 * SW_T_EVENT && offsetof(Scal, smin) % 128 == 0,
+              "words of the device scalars");
 
 // every stage kernel of a halted step returns at once (null: not a step)
 __device__ __forceinline__ bool halted(const Scal *sc) { return sc && sc->halt; }
+
+// The entropy channel (p_S, its flux and its reconstruction) is a ninth of the
+// sweeps' work and traffic, and p_S is zero unless a problem sets it.  While
+// p_S is 0 everywhere and the state is regular (density positive, all of it
+// finite), the step keeps it 0: its flux is 0 and p_S / rho^(gamma-1) is 0.
+// The prologue scans the state (k_scan_entropy) and every cell update reports
+// a p_S that is not 0 or a value that is not finite, from which step on the
+// kernels carry the channel again.  Two words, as the cell update sets one
+// while other blocks of its launch still read the other; k_begin folds them.
+// 256^3 (sweeps i / j / k, cell update, ghost fill): FP64 0.97 / 0.97 / 1.17,
+// 1.59, 0.100 -> 0.86 / 0.86 / 1.15, 1.46, 0.091 ms, FP32-bulk 0.444 / 0.444 /
+// 0.553, 1.01, 0.131 -> 0.390 / 0.392 / 0.533, 0.93, 0.121 ms.
+__device__ __forceinline__ bool carries_entropy(const Scal *sc) { return sc->ent != 0; }
 
 __device__ __forceinline__ double geo3(const Geo &g, int q, int i, int j, int k) {
   return g.g[q][0][i] * g.g[q][1][j] * g.g[q][2][k];
@@ -228,25 +255,41 @@ __device__ __forceinline__ void block_reduce(double dtc, double divb, Scal *sc, 
 // ---------------------------------------------------------------------------
 // Start of a step (one wave per grid): fold the reduction slots into dt, set
 // the AB2 factor and time, dt0 := dt, and reset the slots.
+// Lane q loads word q of the scalars, all in one vector load beside the slots',
+// so the wave waits for memory once (it had chased six scalar loads).  That
+// also orders the reads: a value that is read with a scalar load and replaced
+// with a vector store is only safe if the load has returned before the store
+// is issued, which the compiler does not ensure (some cards read the new dt0).
 __device__ __forceinline__ void begin_step(Scal *sc) {
   const int q = threadIdx.x;  // NSLOT == 64 lanes
-  if (sc->halt) return;
-  if (sc->stop) {  // the previous step ended the run: this step and later ones halt
+  const long long w = ((const long long *)sc)[q < SW_COUNT ? q : 0];
+  const double slot = __longlong_as_double((long long)sc->smin[q]);
+  auto lo = [&](int n) { return __builtin_amdgcn_readlane((int)w, n); };
+  auto hi = [&](int n) { return __builtin_amdgcn_readlane((int)(w >> 32), n); };
+  auto word = [&](int n) { return (long long)hi(n) << 32 | (unsigned int)lo(n); };
+  if (hi(SW_HALT)) return;
+  if (lo(SW_STOP)) {  // the previous step ended the run: this step and later ones halt
     if (q == 0) sc->halt = 1;
     return;
   }
-  const double mn = wave_min(__longlong_as_double((long long)sc->smin[q]));
+  const double dt = wave_min(slot);
   sc->smin[q] = DBL_INF_BITS;
   sc->smax[q] = 0ULL;
+  const double dt0 = __longlong_as_double(word(SW_DT0));
+  const double time = __longlong_as_double(word(SW_TIME)) + dt;
+  long long budget = word(SW_BUDGET);
+  if (budget > 0) budget -= 1;
   if (q == 0) {
-    const double dt = mn;
     sc->dt = dt;
-    sc->time += dt;
-    sc->c = 0.5 * dt / sc->dt0;
     sc->dt0 = dt;
-    sc->steps += 1;
-    if (sc->budget > 0) sc->budget -= 1;
-    if (sc->budget == 0 || sc->time > sc->t_stop || sc->time >= sc->t_event) sc->stop = 1;
+    sc->time = time;
+    sc->c = 0.5 * dt / dt0;
+    sc->budget = budget;
+    sc->steps = word(SW_STEPS) + 1;
+    if (lo(SW_ENT_NEXT)) sc->ent = 1;
+    if (budget == 0 || time > __longlong_as_double(word(SW_T_STOP)) ||
+        time >= __longlong_as_double(word(SW_T_EVENT)))
+      sc->stop = 1;
   }
 }
 
@@ -463,25 +506,17 @@ __device__ __forceinline__ R entropy_over(R ps, R rho) {
 // src/solver_func.c:934-1251) and magnetic stress with B0 cross terms and
 // Boris diffusion (src/solver_func.c:1268-1515).  L/R: rho, v1..3, p, p_S;
 // bl/br: cell-centred B (without B0); Bn: face-normal B at the face.
-// Fo: mass, momentum 1..3, energy, entropy, magnetic stress 1..3.
-template <int D, typename R>
+// Fo: mass, momentum 1..3, energy, entropy, magnetic stress 1..3.  Without the
+// entropy channel (ENT false) L[5], Rs[5] and Fo[5] are not touched.
+template <int D, typename R, bool ENT>
 __device__ __forceinline__ void face_flux(const R L[6], const R Rs[6], const R bl[3],
                                           const R br[3], const R Bn, const R b0[4],
                                           const double CAd, R Fo[9]) {
   const R CA = (R)CAd;
   const R G = (R)GAMMA;
-  const R rl = L[0], rr = Rs[0], pl = L[4], pr = Rs[4], psl = L[5], psr = Rs[5];
+  const R rl = L[0], rr = Rs[0], pl = L[4], pr = Rs[4];
   const R vl[3] = {L[1], L[2], L[3]}, vr[3] = {Rs[1], Rs[2], Rs[3]};
   R csl = qsqrt(qdiv(G * pl, rl)), csr = qsqrt(qdiv(G * pr, rr));
-  // entropy sound speeds, used only squared: with p_S = 0 on both sides (every
-  // problem that does not set it) each square is +0 exactly, and a wave whose
-  // lanes all have it skips the divisions and square roots
-  R cel2 = R(0), cer2 = R(0);
-  if (!(zero_ratio(psl, rl) && zero_ratio(psr, rr))) {
-    const R cel = qsqrt(qdiv(G * psl, rl)), cer = qsqrt(qdiv(G * psr, rr));
-    cel2 = cel * cel;
-    cer2 = cer * cer;
-  }
   // sums of products are written with madd in the reference's order:
   // a + b * c as madd(b, c, a), a - b * c as madd(-b, c, a)
   const R tl[3] = {bl[0] + b0[0], bl[1] + b0[1], bl[2] + b0[2]};
@@ -494,7 +529,6 @@ __device__ __forceinline__ void face_flux(const R L[6], const R Rs[6], const R b
   R vnl = vl[D], vnr = vr[D];
   R VF = fmax(fabs(vnl) + qsqrt(madd(Vel, Vel, csl * csl)),
               fabs(vnr) + qsqrt(madd(Ver, Ver, csr * csr)));
-  R VFe = fmax(fabs(vnl) + qsqrt(madd(Vel, Vel, cel2)), fabs(vnr) + qsqrt(madd(Ver, Ver, cer2)));
   R rvl[3], rvr[3];
 #pragma unroll
   for (int m = 0; m < 3; m++) {
@@ -506,7 +540,6 @@ __device__ __forceinline__ void face_flux(const R L[6], const R Rs[6], const R b
   const R v2r = madd(vr[2], vr[2], madd(vr[1], vr[1], vr[0] * vr[0]));
   R engl = madd(h * rl, v2l, qdiv(pl, R(GAMMA - 1.0)));
   R engr = madd(h * rr, v2r, qdiv(pr, R(GAMMA - 1.0)));
-  R Sl = entropy_over(psl, rl), Sr = entropy_over(psr, rr);
   Fo[0] = h * madd(-VF, rr - rl, rvl[D] + rvr[D]);
 #pragma unroll
   for (int m = 0; m < 3; m++) {
@@ -516,7 +549,22 @@ __device__ __forceinline__ void face_flux(const R L[6], const R Rs[6], const R b
       Fo[1 + m] = h * madd(-VF, rvr[m] - rvl[m], madd(rvr[m], vnr, rvl[m] * vnl));
   }
   Fo[4] = h * madd(-VF, engr - engl, madd(pr, vnr, madd(engr, vnr, madd(pl, vnl, engl * vnl))));
-  Fo[5] = h * madd(-VFe, Sr - Sl, madd(Sr, vnr, Sl * vnl));
+  if constexpr (ENT) {
+    const R psl = L[5], psr = Rs[5];
+    // entropy sound speeds, used only squared: with p_S = 0 on both sides each
+    // square is +0 exactly, and a wave whose lanes all have it skips the
+    // divisions and square roots
+    R cel2 = R(0), cer2 = R(0);
+    if (!(zero_ratio(psl, rl) && zero_ratio(psr, rr))) {
+      const R cel = qsqrt(qdiv(G * psl, rl)), cer = qsqrt(qdiv(G * psr, rr));
+      cel2 = cel * cel;
+      cer2 = cer * cer;
+    }
+    const R VFe =
+        fmax(fabs(vnl) + qsqrt(madd(Vel, Vel, cel2)), fabs(vnr) + qsqrt(madd(Ver, Ver, cer2)));
+    const R Sl = entropy_over(psl, rl), Sr = entropy_over(psr, rr);
+    Fo[5] = h * madd(-VFe, Sr - Sl, madd(Sr, vnr, Sl * vnl));
+  }
 
   const R b0n = b0[3];
   R bsql = madd(R(2), madd(bl[2], b0[2], madd(bl[1], b0[1], bl[0] * b0[0])),
@@ -769,7 +817,7 @@ __device__ __forceinline__ void k_sweep_body(const SweepArgs &a, const int bx, c
 
   R Fo[9], b0[4];
   face_b0<D, R, B0V>(a.b0, a.b0a, g.fs, c, b0);
-  face_flux<D, R>(L, Rs, bl, br, ((const R *)a.B)[D * g.fs + c], b0, g.CA, Fo);
+  face_flux<D, R, true>(L, Rs, bl, br, ((const R *)a.B)[D * g.fs + c], b0, g.CA, Fo);
 #pragma unroll
   for (int m = 0; m < 9; m++) F[m * g.fs + c] = Fo[m];
 }
@@ -810,10 +858,9 @@ __global__ __launch_bounds__(256) void k_sweep_batch(const SweepArgs *__restrict
 // rows per load).  Rows of planes outside [flo0, fhi0] only store the face
 // velocities.  The arithmetic is that of k_sweepk.
 constexpr int KCOL_LDS = 4 * 64 * 9;  // elements of k_kcol's LDS
-template <typename R, bool B0V>
-__device__ __forceinline__ void k_kcol_body(const SweepArgs &a, const int bx, const int by,
+template <typename R, bool B0V, bool ENT>
+__device__ __forceinline__ void k_kcol_part(const SweepArgs &a, const int bx, const int by,
                                        const int bz, R *lds) {
-  if (halted(a.sc)) return;
   (void)by;
   (void)bz;
   R(*sx)[9] = (R(*)[9])lds;  // [row][cell], padded against bank conflicts
@@ -849,6 +896,7 @@ __device__ __forceinline__ void k_kcol_body(const SweepArgs &a, const int bx, co
   R(*sr)[64] = (R(*)[64])(lds + 3 * 64 * 9);
 #pragma unroll 1
   for (int m = 0; m < 9; m++) {
+    if (!ENT && m == 5) continue;
     const R *Pm = m < 6 ? X + m * fs : M + (m - 6) * fs;
     const R *Qm = m < 6 ? Xp + m * fs : Mp + (m - 6) * fs;
     R xv[8], qv[8];
@@ -877,7 +925,7 @@ __device__ __forceinline__ void k_kcol_body(const SweepArgs &a, const int bx, co
   }
   R L[6], Rs[6], bl[3], br[3];
 #pragma unroll
-  for (int m = 0; m < 6; m++) {
+  for (int m = 0; m < (ENT ? 6 : 5); m++) {
     L[m] = sl[m][tx];
     Rs[m] = sr[m][tx];
   }
@@ -893,9 +941,20 @@ __device__ __forceinline__ void k_kcol_body(const SweepArgs &a, const int bx, co
   if (!full) return;
   R Fo[9], b0[4];
   face_b0<2, R, B0V>(a.b0, a.b0a, fs, c, b0);
-  face_flux<2, R>(L, Rs, bl, br, ((const R *)a.B)[2 * fs + c], b0, g.CA, Fo);
+  face_flux<2, R, ENT>(L, Rs, bl, br, ((const R *)a.B)[2 * fs + c], b0, g.CA, Fo);
 #pragma unroll
-  for (int m = 0; m < 9; m++) st_nt(F + m * fs + c, Fo[m]);
+  for (int m = 0; m < 9; m++)
+    if (ENT || m != 5) st_nt(F + m * fs + c, Fo[m]);
+}
+
+template <typename R, bool B0V>
+__device__ __forceinline__ void k_kcol_body(const SweepArgs &a, const int bx, const int by,
+                                       const int bz, R *lds) {
+  if (halted(a.sc)) return;
+  if (carries_entropy(a.sc))
+    k_kcol_part<R, B0V, true>(a, bx, by, bz, lds);
+  else
+    k_kcol_part<R, B0V, false>(a, bx, by, bz, lds);
 }
 
 template <typename R, bool B0V>
@@ -969,10 +1028,9 @@ __device__ __forceinline__ void march_lr(const Window<NF, R> &w, int m, const R 
   pdm_pair(fl, fr, w.x[m][0], w.x[m][1], w.x[m][2], w.x[m][3], T, L, Rr);
 }
 
-template <int D, typename R, bool B0V, bool UT>
-__device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, const int by,
+template <int D, typename R, bool B0V, bool UT, bool ENT>
+__device__ __forceinline__ void k_march_part(const SweepArgs &a, const int bx, const int by,
                                         const int bz) {
-  if (halted(a.sc)) return;
   constexpr int RA = D == 0 ? 1 : 0;  // row axis
   const Grid &g = a.g;
   (void)by;
@@ -995,30 +1053,32 @@ __device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, c
   R *F = (R *)a.F, *V = (R *)a.V;
   const R *X = (const R *)a.X, *Xp = (const R *)a.Xp;
   if (r >= a.flo[RA] && r <= a.fhi[RA]) {
-    const R *P[9], *Q[9];
+    // fields: density, velocity, pressure (and p_S), then the cell-centred B
+    constexpr int NX = ENT ? 6 : 5, NF = NX + 3;
+    const R *P[NF], *Q[NF];
 #pragma unroll
-    for (int m = 0; m < 6; m++) {
+    for (int m = 0; m < NX; m++) {
       P[m] = X + m * fs;
       Q[m] = Xp + m * fs;
     }
 #pragma unroll
     for (int m = 0; m < 3; m++) {
-      P[6 + m] = (const R *)a.M + m * fs;
-      Q[6 + m] = (const R *)a.Mp + m * fs;
+      P[NX + m] = (const R *)a.M + m * fs;
+      Q[NX + m] = (const R *)a.Mp + m * fs;
     }
-    Window<9, R> w;
+    Window<NF, R> w;
 #pragma unroll
-    for (int p = 0; p < 7; p++) march_load<9, R, R>(w, P, Q, c + (p - 4) * sd, cc, p);
+    for (int p = 0; p < 7; p++) march_load<NF, R, R>(w, P, Q, c + (p - 4) * sd, cc, p);
     // FP64: the raw values of the cell entering the window and the
     // face-normal B are loaded one face ahead, so their HBM latency overlaps
     // the previous face's arithmetic (one wave per SIMD leaves no other wave
     // to cover it).  FP32 keeps the plain order, which measured faster.
     constexpr bool AHEAD = sizeof(R) == 8;
     const R *Bd = (const R *)a.B + D * fs;
-    R nx[9], nq[9], nb = R(0);
+    R nx[NF], nq[NF], nb = R(0);
     if constexpr (AHEAD) {
 #pragma unroll
-      for (int m = 0; m < 9; m++) {
+      for (int m = 0; m < NF; m++) {
         nx[m] = P[m][c + 3 * sd];
         nq[m] = Q[m][c + 3 * sd];
       }
@@ -1028,21 +1088,21 @@ __device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, c
       R bn;
       if constexpr (AHEAD) {
 #pragma unroll
-        for (int m = 0; m < 9; m++) {
+        for (int m = 0; m < NF; m++) {
           w.h[m][7] = half_step(nx[m], nq[m], cc);
           w.x[m][5] = nx[m];
         }
         bn = nb;
         if (f + 1 < f1) {
 #pragma unroll
-          for (int m = 0; m < 9; m++) {
+          for (int m = 0; m < NF; m++) {
             nx[m] = P[m][c + 4 * sd];
             nq[m] = Q[m][c + 4 * sd];
           }
           nb = Bd[c + sd];
         }
       } else {
-        march_load<9, R, R>(w, P, Q, c + 3 * sd, cc, 7);
+        march_load<NF, R, R>(w, P, Q, c + 3 * sd, cc, 7);
         bn = Bd[c];
       }
       R Tu[UT ? GK_RECW_STRIDE : 1];
@@ -1053,16 +1113,17 @@ __device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, c
       }
       R L[6], Rs[6], bl[3], br[3];
 #pragma unroll
-      for (int m = 0; m < 6; m++) march_lr(w, m, Tf, L[m], Rs[m]);
+      for (int m = 0; m < NX; m++) march_lr(w, m, Tf, L[m], Rs[m]);
 #pragma unroll
-      for (int m = 0; m < 3; m++) march_lr(w, 6 + m, Tf, bl[m], br[m]);
+      for (int m = 0; m < 3; m++) march_lr(w, NX + m, Tf, bl[m], br[m]);
       st_nt(V + c, R(0.5) * (L[va] + Rs[va]));
       st_nt(V + fs + c, R(0.5) * (L[vb] + Rs[vb]));
       R Fo[9], b0[4];
       face_b0<D, R, B0V>(a.b0, a.b0a, fs, c, b0);
-      face_flux<D, R>(L, Rs, bl, br, bn, b0, g.CA, Fo);
+      face_flux<D, R, ENT>(L, Rs, bl, br, bn, b0, g.CA, Fo);
 #pragma unroll
-      for (int m = 0; m < 9; m++) st_nt(F + m * fs + c, Fo[m]);
+      for (int m = 0; m < 9; m++)
+        if (ENT || m != 5) st_nt(F + m * fs + c, Fo[m]);
       march_shift(w);
       c += sd;
       T += tstep;
@@ -1094,7 +1155,27 @@ __device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, c
 }
 
 template <int D, typename R, bool B0V, bool UT>
-__global__ __launch_bounds__(256) void k_march(SweepArgs a, int gx, int gy, int gz) {
+__device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, const int by,
+                                        const int bz) {
+  if (halted(a.sc)) return;
+  if (carries_entropy(a.sc))
+    k_march_part<D, R, B0V, UT, true>(a, bx, by, bz);
+  else
+    k_march_part<D, R, B0V, UT, false>(a, bx, by, bz);
+}
+
+// Waves per SIMD a march is held to: those each of its two bodies (with and
+// without the entropy channel) reaches alone.  Without the bound the compiler
+// keeps addresses of both live and the FP32-bulk march ends at 265 registers,
+// one wave.
+template <typename R>
+struct MarchWaves {
+  static constexpr int n = sizeof(R) == 4 ? 2 : 1;
+};
+
+template <int D, typename R, bool B0V, bool UT>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(MarchWaves<R>::n))) void k_march(SweepArgs a, int gx, int gy, int gz) {
   int bx, by, bz;
   if (!xcd_block<true>(gx, gy, gz, bx, by, bz)) return;
   k_march_body<D, R, B0V, UT>(a, bx, by, bz);
@@ -1102,7 +1183,8 @@ __global__ __launch_bounds__(256) void k_march(SweepArgs a, int gx, int gy, int 
 
 // one launch for many grids: block w runs work-list entry w (argument set, block)
 template <int D, typename R, bool B0V, bool UT>
-__global__ __launch_bounds__(256) void k_march_batch(const SweepArgs *__restrict__ args,
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(MarchWaves<R>::n))) void k_march_batch(const SweepArgs *__restrict__ args,
                                                     const WorkItem *__restrict__ work, int nwork) {
   int w;
   if (!xcd_item(nwork, w)) return;
@@ -1124,10 +1206,9 @@ constexpr int KSPAN = 72;
 constexpr int SWEEPK_LDS = 2 * 9 * KSPAN;  // elements of k_sweepk's LDS
 constexpr int CELL_CHUNK = 1;  // cells each thread of the cell update walks along i
 
-template <typename R, bool B0V>
-__device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, const int by,
+template <typename R, bool B0V, bool ENT>
+__device__ __forceinline__ void k_sweepk_part(const SweepArgs &a, const int bx, const int by,
                                          const int bz, R *lds) {
-  if (halted(a.sc)) return;
   R(*sh)[KSPAN] = (R(*)[KSPAN])lds;
   R(*sx)[KSPAN] = (R(*)[KSPAN])(lds + 9 * KSPAN);
   const Grid &g = a.g;
@@ -1178,9 +1259,11 @@ __device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, 
   };
   if (full) {
 #pragma unroll
-    for (int m = 0; m < 9; m++) fetch(m);
+    for (int m = 0; m < 9; m++)
+      if (ENT || m != 5) fetch(m);
 #pragma unroll
-    for (int m = 0; m < 9; m++) stage(m);
+    for (int m = 0; m < 9; m++)
+      if (ENT || m != 5) stage(m);
   } else {
     fetch(3);
     fetch(1);
@@ -1209,16 +1292,27 @@ __device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, 
   }
   R L[6], Rs[6], bl[3], br[3];
 #pragma unroll
-  for (int m = 0; m < 6; m++) lr(m, L[m], Rs[m]);
+  for (int m = 0; m < (ENT ? 6 : 5); m++) lr(m, L[m], Rs[m]);
 #pragma unroll
   for (int m = 0; m < 3; m++) lr(6 + m, bl[m], br[m]);
   st_nt(V + c, R(0.5) * (L[3] + Rs[3]));
   st_nt(V + fs + c, R(0.5) * (L[1] + Rs[1]));
   R Fo[9], b0[4];
   face_b0<2, R, B0V>(a.b0, a.b0a, fs, c, b0);
-  face_flux<2, R>(L, Rs, bl, br, ((const R *)a.B)[2 * fs + c], b0, g.CA, Fo);
+  face_flux<2, R, ENT>(L, Rs, bl, br, ((const R *)a.B)[2 * fs + c], b0, g.CA, Fo);
 #pragma unroll
-  for (int m = 0; m < 9; m++) st_nt(F + m * fs + c, Fo[m]);
+  for (int m = 0; m < 9; m++)
+    if (ENT || m != 5) st_nt(F + m * fs + c, Fo[m]);
+}
+
+template <typename R, bool B0V>
+__device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, const int by,
+                                         const int bz, R *lds) {
+  if (halted(a.sc)) return;
+  if (carries_entropy(a.sc))
+    k_sweepk_part<R, B0V, true>(a, bx, by, bz, lds);
+  else
+    k_sweepk_part<R, B0V, false>(a, bx, by, bz, lds);
 }
 
 template <typename R, bool B0V>
@@ -1824,6 +1918,7 @@ template <typename R, bool B0V>
 __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, const int by,
                                        const int bz) {
   if (halted(a.sc)) return;
+  const bool ent = carries_entropy(a.sc);
   const Grid &g = a.g;
   const Geo &G = a.geo;
   int k, j;
@@ -1839,6 +1934,18 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
   for (int i = i0; i < i1; i++) {
     const long c = i * g.st[0] + j * g.st[1] + k;
     const int idx[3] = {i, j, k};
+    // the entropy channel's inputs, first, so that the loads of every other
+    // input follow in one block
+    R f5[3][2] = {};
+    double x5 = 0.0;
+    if (ent) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        f5[d][0] = ((const R *)a.F[d])[5 * g.fs + c];
+        f5[d][1] = ((const R *)a.F[d])[5 * g.fs + c + g.st[d]];
+      }
+      x5 = ld_nt(a.X + 5 * g.fs + c);
+    }
     const double dt = a.sc->dt;
     const double CA = g.CA;
     const double V = geo3(G, GK_G_VOL, i, j, k);
@@ -1864,11 +1971,20 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
       const long sd = g.st[d];
 #pragma unroll
       for (int m = 0; m < 9; m++) {
+        if (m == 5) continue;  // entropy: below
         double v = (double)Fd[m * g.fs + c + sd] * A1[d] - (double)Fd[m * g.fs + c] * A0[d];
         // FP64 divides every term by V as the reference does; FP32-bulk
         // (fluxes already rounded to FP32) multiplies by 1/V
         v = sizeof(R) == 4 ? v * iV : v / V;
         dU[m] = d == 0 ? v : dU[m] + v;
+      }
+    }
+    if (ent) {
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        double v = (double)f5[d][1] * A1[d] - (double)f5[d][0] * A0[d];
+        v = sizeof(R) == 4 ? v * iV : v / V;
+        dU[5] = d == 0 ? v : dU[5] + v;
       }
     }
     // background field at the cell: Lorentz force, cell-centre B0 and the
@@ -1895,7 +2011,8 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
 
     double x[6];
 #pragma unroll
-    for (int m = 0; m < 6; m++) x[m] = ld_nt(a.X + m * g.fs + c);
+    for (int m = 0; m < 5; m++) x[m] = ld_nt(a.X + m * g.fs + c);
+    x[5] = x5;
     double bold[3];
 #pragma unroll
     for (int m = 0; m < 3; m++) bold[m] = (double)ld_nt((const R *)a.M + m * g.fs + c);
@@ -1915,9 +2032,9 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
     double SH[3] = {0.0, 0.0, 0.0}, SB[3] = {0.0, 0.0, 0.0};
     if (a.spherical) {
       const double cc = a.sc->c;
-      double xp[6];
+      double xp[5];
 #pragma unroll
-      for (int m = 0; m < 6; m++) xp[m] = a.Xp[m * g.fs + c];
+      for (int m = 0; m < 5; m++) xp[m] = a.Xp[m * g.fs + c];
       double rh = x[0] + cc * (x[0] - xp[0]);
       double v2h = x[2] + cc * (x[2] - xp[2]);
       double v3h = x[3] + cc * (x[3] - xp[3]);
@@ -1965,10 +2082,10 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
 #pragma unroll
     for (int m = 0; m < 3; m++) ru[m] = ru0[m] - dt * dU[1 + m] + dt * SH[m];
     double eng = eng0 - dt * dU[4];
-    double ent = ent0 - dt * dU[5];
+    double entn = ent0 - dt * dU[5];
     double v1 = ru[0] / rho, v2 = ru[1] / rho, v3 = ru[2] / rho;
     double p = (eng - 0.5 * (v1 * v1 + v2 * v2 + v3 * v3) * rho) * (GAMMA - 1.0);
-    double ps = entropy_times(ent, rho);
+    double ps = entropy_times(entn, rho);
     double rhof = rho;
     if (rhof < a.rho_floor) {
       rhof = a.rho_floor;
@@ -1999,13 +2116,16 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
     }
     double out[6] = {rhof, vn[0], vn[1], vn[2], p, ps};
 #pragma unroll
-    for (int m = 0; m < 6; m++) {
-      st_nt(a.Xn + m * g.fs + c, out[m]);
-      bad |= !isfinite(out[m]);
-    }
+    for (int m = 0; m < 5; m++) st_nt(a.Xn + m * g.fs + c, out[m]);
+#pragma unroll
+    for (int m = 0; m < 6; m++) bad |= !isfinite(out[m]);
     if (a.Xn32) {
 #pragma unroll
-      for (int m = 0; m < 6; m++) st_nt(a.Xn32 + m * g.fs + c, (float)out[m]);
+      for (int m = 0; m < 5; m++) st_nt(a.Xn32 + m * g.fs + c, (float)out[m]);
+    }
+    if (ent || !(ps == 0.0)) {  // not carried: the buffers hold 0 where nothing is stored
+      st_nt(a.Xn + 5 * g.fs + c, ps);
+      if (a.Xn32) st_nt(a.Xn32 + 5 * g.fs + c, (float)ps);
     }
     // cell-centred B at n+1 (the ghost cells' is formed after the ghost fill)
 #pragma unroll
@@ -2029,7 +2149,10 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
       divb = fmax(divb, adb);
   }
   block_reduce(dtc, divb, a.sc, bx * 31 + by * 7 + bz);
-  if (bad) atomicOr(&a.sc->nanflag, 1u);
+  if (bad) {
+    atomicOr(&a.sc->nanflag, 1u);
+    atomicOr(&a.sc->ent_next, 1u);
+  }
 }
 
 template <typename R, bool B0V>
@@ -2293,12 +2416,16 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
     if (pb[f]) m[2] = pole_k(g, k);
     sb[f] = m[0] * g.st[0] + m[1] * g.st[1] + m[2];
   }
+  // p_S moves only while the step carries it, or where this step's cell update
+  // has just written one that is not 0 (everything outside a step)
+  const int nx = !a.sc || a.sc->ent || a.sc->ent_next ? 6 : 5;
   double xv[6], bv[3];
   float xw[6], bw[3];
   if (sx != c) {
     if (a.X) {
 #pragma unroll
-      for (int m = 0; m < 6; m++) xv[m] = a.X[m * g.fs + sx];
+      for (int m = 0; m < 6; m++)
+        if (m < nx) xv[m] = a.X[m * g.fs + sx];
       if (px) {
         xv[2] = -xv[2];
         xv[3] = -xv[3];
@@ -2309,7 +2436,8 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
     }
     if (a.X32) {
 #pragma unroll
-      for (int m = 0; m < 6; m++) xw[m] = a.X32[m * g.fs + sx];
+      for (int m = 0; m < 6; m++)
+        if (m < nx) xw[m] = a.X32[m * g.fs + sx];
       if (px) {
         xw[2] = -xw[2];
         xw[3] = -xw[3];
@@ -2336,7 +2464,7 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
     }
   }
   if (sx != c || fx) {
-    const int nm = sx != c ? 6 : 5;  // p_S mapped to itself is left alone
+    const int nm = sx != c ? nx : 5;  // p_S mapped to itself is left alone
     if (a.X) {
 #pragma unroll
       for (int m = 0; m < 6; m++)
@@ -2425,6 +2553,30 @@ __device__ __forceinline__ void k_mags_body(const MagsArgs &a, const int bx, con
     if (a.M) a.M[m * g.fs + c] = b[m];
     if (a.M32) a.M32[m * g.fs + c] = (float)b[m];
   }
+}
+
+// Whether a state needs the entropy channel (carries_entropy): p_S not 0
+// somewhere, or a value out of the range in which the step surely keeps it 0
+// (density positive, everything finite, in the FP32 copies too), over the
+// points the stencils read
+struct ScanArgs {
+  Grid g;
+  const double *X[2], *M[2];  // both time levels
+  Scal *sc;
+};
+
+__global__ __launch_bounds__(256) void k_scan_entropy(ScanArgs a) {
+  const Grid &g = a.g;
+  int k, j;
+  if (!row_point(0, g.N[2] - 2, 0, g.N[1] - 2, blockIdx.x, k, j)) return;
+  const long c = blockIdx.z * g.st[0] + j * g.st[1] + k;
+  bool regular = true;
+  for (int t = 0; t < 2; t++) {
+    for (int m = 0; m < 5; m++) regular = regular && fabs(a.X[t][m * g.fs + c]) < 1e30;
+    for (int m = 0; m < 3; m++) regular = regular && fabs(a.M[t][m * g.fs + c]) < 1e15;
+    regular = regular && a.X[t][c] > 1e-30 && a.X[t][5 * g.fs + c] == 0.0;
+  }
+  if (!regular) atomicOr(&a.sc->ent, 1u);
 }
 
 // reference layout (pitch NK) <-> padded device layout (pitch KP)
@@ -3705,6 +3857,14 @@ extern "C" int gk_prologue(gk_solver *s, double dt0_restart) {
   z.t_event = INFINITY;
   memcpy(pin, &z, sizeof z);
   HIPCHK(hipMemcpyAsync(s->sc, pin, sizeof(Scal), hipMemcpyHostToDevice, s->stream));
+  ScanArgs sa;
+  sa.g = s->g;
+  sa.X[0] = s->X[s->cur];
+  sa.X[1] = s->X[1 - s->cur];
+  sa.M[0] = s->M[s->b_0];
+  sa.M[1] = s->M[s->b_m1];
+  sa.sc = s->sc;
+  k_scan_entropy<<<mags_grid(s->g), dim3(64, 4), 0, s->stream>>>(sa);
   DtArgs a;
   a.g = s->g;
   a.geo = s->geo;
@@ -4592,6 +4752,13 @@ extern "C" int gk_debug_fetch(gk_solver *s, int which, int field, double *host) 
     esz = sizeof(double);
   }
   if (!src) return GK_ERR_ARG;
+  if (which < 3 && field == 5) {  // the entropy flux is 0 where the steps do not carry it
+    double sc6[6];
+    const int rc = gk_get_scalars(s, sc6);
+    if (rc != GK_OK) return rc;
+    if (!((const Scal *)(s->ctl_host + 2))->ent)
+      HIPCHK(hipMemsetAsync((char *)s->F[which] + field * fb, 0, fb, s->stream));
+  }
   if (esz == sizeof(double)) {
     int rc = copy_out(s, host, (const double *)src);
     if (rc != GK_OK) return rc;
