@@ -750,6 +750,7 @@ struct SweepArgs {
   int lo[3], hi[3];
   int flo[3], fhi[3];    // range where the full flux is needed
   int nch;               // marching sweeps: near-equal chunks of the march range
+  int rp;                // k sweep: rows packed into a tile (1: none)
   int gap;               // velocity strips: strip-axis indices from NGH on are
                          // shifted by gap (both ghost strips in one box)
 };
@@ -767,18 +768,14 @@ __device__ __forceinline__ void globalize(SweepArgs &a) {
   gptr(a.sc);
 }
 
-// Direct sweep for the velocity-only strips of the j sweep (k in the four
-// ghost layers on either side).  Each thread reads its eight stencil cells;
-// the points of the launch box are walked k fastest, then j, then i, 256 per
-// block.
-template <int D, typename R, bool B0V>
-__device__ __forceinline__ void k_sweep_body(const SweepArgs &a, const int bx, const int by,
-                                        const int bz) {
-  if (halted(a.sc)) return;
-  (void)by;
-  (void)bz;
+// Direct sweep, one face per thread, for the velocity-only strips of the i and
+// j sweeps (ghost rows and columns).  Each thread reads its eight stencil
+// cells; the points of the launch box are walked k fastest, then j, then i,
+// 256 per block.
+template <int D, typename R>
+__device__ __forceinline__ void k_strip_part(const SweepArgs &a, const int bx, const int ty) {
   const int W = a.hi[2] - a.lo[2] + 1, H = a.hi[1] - a.lo[1] + 1;
-  const int p = bx * 256 + threadIdx.y * 64 + threadIdx.x;
+  const int p = bx * 256 + ty * 64 + threadIdx.x;
   const int t = p / W;
   int k = a.lo[2] + (p - t * W);
   int j = a.lo[1] + t % H;
@@ -788,49 +785,38 @@ __device__ __forceinline__ void k_sweep_body(const SweepArgs &a, const int bx, c
   if (D == 1 && k >= NGH) k += a.gap;
   const Grid &g = a.g;
   const long c = i * g.st[0] + j * g.st[1] + k;
-  const long sd = g.st[D];
   const int idx[3] = {i, j, k};
-  const int f = idx[D];
-  const bool full = i >= a.flo[0] && i <= a.fhi[0] && j >= a.flo[1] && j <= a.fhi[1] &&
-                    k >= a.flo[2] && k <= a.fhi[2];
   const R cc = (R)a.sc->c;
-  const R *T = rtab<D, R>(a.geo, f, idx);
-  R *F = (R *)a.F, *V = (R *)a.V;
-
-  // velocity components that feed the edge fields: D=0 (v1,v2), 1 (v2,v3), 2 (v3,v1)
-  constexpr int va = D == 0 ? 1 : (D == 1 ? 2 : 3);
-  constexpr int vb = D == 0 ? 2 : (D == 1 ? 3 : 1);
-  R L[6], Rs[6];
-#pragma unroll
-  for (int m = 0; m < 6; m++) {
-    if (!full && m != va && m != vb) continue;
-    recon((const R *)a.X + m * g.fs, (const R *)a.Xp + m * g.fs, c, sd, cc, T, L[m], Rs[m]);
-  }
-  V[c] = R(0.5) * (L[va] + Rs[va]);
-  V[g.fs + c] = R(0.5) * (L[vb] + Rs[vb]);
-  if (!full) return;
-
-  R bl[3], br[3];
-#pragma unroll
-  for (int m = 0; m < 3; m++)
-    recon((const R *)a.M + m * g.fs, (const R *)a.Mp + m * g.fs, c, sd, cc, T, bl[m], br[m]);
-
-  R Fo[9], b0[4];
-  face_b0<D, R, B0V>(a.b0, a.b0a, g.fs, c, b0);
-  face_flux<D, R, true>(L, Rs, bl, br, ((const R *)a.B)[D * g.fs + c], b0, g.CA, Fo);
-#pragma unroll
-  for (int m = 0; m < 9; m++) F[m * g.fs + c] = Fo[m];
+  const R *T = rtab<D, R>(a.geo, idx[D], idx);
+  R *V = (R *)a.V;
+  // velocity components that feed the edge fields: D=0 (v1,v2), 1 (v2,v3)
+  constexpr int va = D == 0 ? 1 : 2, vb = D == 0 ? 2 : 3;
+  const R *X = (const R *)a.X, *Xp = (const R *)a.Xp;
+  R l[2], r[2];
+  recon(X + va * g.fs, Xp + va * g.fs, c, g.st[D], cc, T, l[0], r[0]);
+  recon(X + vb * g.fs, Xp + vb * g.fs, c, g.st[D], cc, T, l[1], r[1]);
+  V[c] = R(0.5) * (l[0] + r[0]);
+  V[g.fs + c] = R(0.5) * (l[1] + r[1]);
 }
 
-template <int D, typename R, bool B0V>
+template <int D, typename R>
+__device__ __forceinline__ void k_sweep_body(const SweepArgs &a, const int bx, const int by,
+                                        const int bz) {
+  (void)by;
+  (void)bz;
+  if (halted(a.sc)) return;
+  k_strip_part<D, R>(a, bx, threadIdx.y);
+}
+
+template <int D, typename R>
 __global__ __launch_bounds__(256) void k_sweep(SweepArgs a, int gx, int gy, int gz) {
   int bx, by, bz;
   if (!xcd_block<false>(gx, gy, gz, bx, by, bz)) return;
-  k_sweep_body<D, R, B0V>(a, bx, by, bz);
+  k_sweep_body<D, R>(a, bx, by, bz);
 }
 
 // one launch for many grids: block w runs work-list entry w (argument set, block)
-template <int D, typename R, bool B0V>
+template <int D, typename R>
 __global__ __launch_bounds__(256) void k_sweep_batch(const SweepArgs *__restrict__ args,
                                                     const WorkItem *__restrict__ work, int nwork) {
   int w;
@@ -840,7 +826,7 @@ __global__ __launch_bounds__(256) void k_sweep_batch(const SweepArgs *__restrict
   const int bx = __builtin_amdgcn_readfirstlane(work[w].bx);
   const int by = __builtin_amdgcn_readfirstlane(work[w].by);
   const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
-  k_sweep_body<D, R, B0V>(batch_args(args, arg), bx, by, bz);
+  k_sweep_body<D, R>(batch_args(args, arg), bx, by, bz);
 }
 
 // Marching sweep along D = 0 (i) or 1 (j).  Lanes run along k (coalesced),
@@ -982,10 +968,11 @@ __global__ __launch_bounds__(64) void k_kcol_batch(const SweepArgs *__restrict__
 // row by row, k fastest, 256 points per block (bx), so a k extent that is not
 // a multiple of 64 (257 faces or edges, small grids) does not leave waves
 // mostly empty; the lanes of a wave may span two rows.
+// Launches of one-wave blocks pass the wave of the 256 points (ty).
 __device__ __forceinline__ bool row_point(int klo, int khi, int rlo, int rhi, int bx, int &k,
-                                          int &r) {
+                                          int &r, int ty = -1) {
   const int wk = khi - klo + 1;
-  const int p = bx * 256 + threadIdx.y * 64 + threadIdx.x;
+  const int p = bx * 256 + (ty < 0 ? (int)threadIdx.y : ty) * 64 + threadIdx.x;
   const int q = p / wk;
   r = rlo + q;
   k = klo + (p - q * wk);
@@ -1029,13 +1016,12 @@ __device__ __forceinline__ void march_lr(const Window<NF, R> &w, int m, const R 
 }
 
 template <int D, typename R, bool B0V, bool UT, bool ENT>
-__device__ __forceinline__ void k_march_part(const SweepArgs &a, const int bx, const int by,
+__device__ __forceinline__ void k_march_part(const SweepArgs &a, const int bx, const int ty,
                                         const int bz) {
   constexpr int RA = D == 0 ? 1 : 0;  // row axis
   const Grid &g = a.g;
-  (void)by;
   int k, r;
-  if (!row_point(a.lo[2], a.hi[2], a.lo[RA], a.hi[RA], bx, k, r)) return;
+  if (!row_point(a.lo[2], a.hi[2], a.lo[RA], a.hi[RA], bx, k, r, ty)) return;
   int f0, f1;
   march_range(a.lo[D], a.hi[D], a.nch, bz, f0, f1);
   int idx[3];
@@ -1157,11 +1143,12 @@ __device__ __forceinline__ void k_march_part(const SweepArgs &a, const int bx, c
 template <int D, typename R, bool B0V, bool UT>
 __device__ __forceinline__ void k_march_body(const SweepArgs &a, const int bx, const int by,
                                         const int bz) {
+  (void)by;
   if (halted(a.sc)) return;
   if (carries_entropy(a.sc))
-    k_march_part<D, R, B0V, UT, true>(a, bx, by, bz);
+    k_march_part<D, R, B0V, UT, true>(a, bx, threadIdx.y, bz);
   else
-    k_march_part<D, R, B0V, UT, false>(a, bx, by, bz);
+    k_march_part<D, R, B0V, UT, false>(a, bx, threadIdx.y, bz);
 }
 
 // Waves per SIMD a march is held to: those each of its two bodies (with and
@@ -1203,6 +1190,11 @@ __global__ __launch_bounds__(256)
 // write, so the wave waits for memory once, not once per field.  Planes i
 // outside [flo0, fhi0] only form the face-averaged velocities (v3, v1).
 constexpr int KSPAN = 72;
+// rows of up to 32 faces are packed, several to a tile (k_sweepk_pack), as many
+// as 64 faces and PACKSPAN cells (7 more than faces per row) allow; PACKSPAN
+// keeps the tile's LDS below what KCOL_LDS takes
+constexpr int PACKSPAN = 112;
+constexpr int PACKK_LDS = 2 * 9 * PACKSPAN;
 constexpr int SWEEPK_LDS = 2 * 9 * KSPAN;  // elements of k_sweepk's LDS
 constexpr int CELL_CHUNK = 1;  // cells each thread of the cell update walks along i
 
@@ -1305,6 +1297,89 @@ __device__ __forceinline__ void k_sweepk_part(const SweepArgs &a, const int bx, 
     if (ENT || m != 5) st_nt(F + m * fs + c, Fo[m]);
 }
 
+// k sweep of short rows (32 faces or fewer): a wave covers rp whole rows of W
+// faces, their W + 7 cells staged one row after the other.  One row
+// per wave left 55 of 64 lanes idle at nk = 8 (128x128x8 FP64: 0.059 -> 0.025
+// ms).
+template <typename R, bool B0V, bool ENT>
+__device__ __forceinline__ void k_sweepk_pack(const SweepArgs &a, const int tile, R *lds) {
+  R(*sh)[PACKSPAN] = (R(*)[PACKSPAN])lds;
+  R(*sx)[PACKSPAN] = (R(*)[PACKSPAN])(lds + 9 * PACKSPAN);
+  const Grid &g = a.g;
+  const int W = a.hi[2] - a.lo[2] + 1, S = W + 7, H = a.hi[1] - a.lo[1] + 1;
+  const int nrow = H * (a.hi[0] - a.lo[0] + 1), row0 = tile * a.rp;
+  const int tx = threadIdx.x;
+  const long fs = g.fs;
+  const R cc = (R)a.sc->c;
+  R *F = (R *)a.F, *V = (R *)a.V;
+  const R *X = (const R *)a.X, *Xp = (const R *)a.Xp;
+  const R *M = (const R *)a.M, *Mp = (const R *)a.Mp;
+  auto field = [&](int m) { return m < 6 ? X + m * fs : M + (m - 6) * fs; };
+  auto field_p = [&](int m) { return m < 6 ? Xp + m * fs : Mp + (m - 6) * fs; };
+  // the rows' planes are full or velocity-only, some of each where the tile
+  // crosses from one kind to the other
+  const int i0 = a.lo[0] + row0 / H, i1 = a.lo[0] + (min(row0 + a.rp, nrow) - 1) / H;
+  const bool any_full = i1 >= a.flo[0] && i0 <= a.fhi[0];
+  // lane tx stages cells tx and tx + 64 of the tile
+  R xv[9][2], pv[9][2];
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const int q = tx + 64 * s, rr = q / S, row = min(row0 + rr, nrow - 1);
+    if (q < a.rp * S) {
+      const long o = (long)(a.lo[0] + row / H) * g.st[0] + (long)(a.lo[1] + row % H) * g.st[1] +
+                     a.lo[2] - 4 + (q - rr * S);
+#pragma unroll
+      for (int m = 0; m < 9; m++)
+        if ((ENT || m != 5) && (any_full || m == 3 || m == 1)) {
+          xv[m][s] = field(m)[o];
+          pv[m][s] = field_p(m)[o];
+        }
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < 2; s++) {
+    const int q = tx + 64 * s;
+    if (q < a.rp * S) {
+#pragma unroll
+      for (int m = 0; m < 9; m++)
+        if ((ENT || m != 5) && (any_full || m == 3 || m == 1)) {
+          sh[m][q] = half_step(xv[m][s], pv[m][s], cc);
+          sx[m][q] = xv[m][s];
+        }
+    }
+  }
+  __syncthreads();
+  const int rr = tx / W, f = tx - rr * W, row = row0 + rr;
+  if (rr >= a.rp || row >= nrow) return;
+  const int i = a.lo[0] + row / H, j = a.lo[1] + row % H, k = a.lo[2] + f;
+  const int idx[3] = {i, j, k};
+  const R *T = rtab<2, R>(a.geo, k, idx);
+  const long c = (long)i * g.st[0] + (long)j * g.st[1] + k;
+  const int b = rr * S + f;
+  auto lr = [&](int m, R &L, R &Rr) {
+    R fl, fr;
+    interpolate(&sh[m][b], T, fl, fr);
+    pdm_pair(fl, fr, sx[m][b + 2], sx[m][b + 3], sx[m][b + 4], sx[m][b + 5], T, L, Rr);
+  };
+  R L[6], Rs[6], bl[3], br[3];
+  lr(3, L[3], Rs[3]);
+  lr(1, L[1], Rs[1]);
+  st_nt(V + c, R(0.5) * (L[3] + Rs[3]));
+  st_nt(V + fs + c, R(0.5) * (L[1] + Rs[1]));
+  if (i < a.flo[0] || i > a.fhi[0]) return;
+#pragma unroll
+  for (int m = 0; m < (ENT ? 6 : 5); m++)
+    if (m != 3 && m != 1) lr(m, L[m], Rs[m]);
+#pragma unroll
+  for (int m = 0; m < 3; m++) lr(6 + m, bl[m], br[m]);
+  R Fo[9], b0[4];
+  face_b0<2, R, B0V>(a.b0, a.b0a, fs, c, b0);
+  face_flux<2, R, ENT>(L, Rs, bl, br, ((const R *)a.B)[2 * fs + c], b0, g.CA, Fo);
+#pragma unroll
+  for (int m = 0; m < 9; m++)
+    if (ENT || m != 5) st_nt(F + m * fs + c, Fo[m]);
+}
+
 template <typename R, bool B0V>
 __device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, const int by,
                                          const int bz, R *lds) {
@@ -1313,6 +1388,39 @@ __device__ __forceinline__ void k_sweepk_body(const SweepArgs &a, const int bx, 
     k_sweepk_part<R, B0V, true>(a, bx, by, bz, lds);
   else
     k_sweepk_part<R, B0V, false>(a, bx, by, bz, lds);
+}
+
+// The packed tiles have kernels of their own: as a branch of the plain tiles'
+// they cost those 4 % (256^3 FP32-bulk 0.537 -> 0.561 ms).
+template <typename R, bool B0V>
+__device__ __forceinline__ void k_packk_body(const SweepArgs &a, const int bx, const int by,
+                                        const int bz, R *lds) {
+  (void)by;
+  (void)bz;
+  if (halted(a.sc)) return;
+  if (carries_entropy(a.sc))
+    k_sweepk_pack<R, B0V, true>(a, bx, lds);
+  else
+    k_sweepk_pack<R, B0V, false>(a, bx, lds);
+}
+
+template <typename R, bool B0V>
+__global__ __launch_bounds__(64) void k_packk(SweepArgs a, int gx, int gy, int gz) {
+  int bx, by, bz;
+  if (!xcd_block<false>(gx, gy, gz, bx, by, bz)) return;
+  __shared__ R lds[PACKK_LDS];
+  k_packk_body<R, B0V>(a, bx, by, bz, lds);
+}
+
+template <typename R, bool B0V>
+__global__ __launch_bounds__(64) void k_packk_batch(const SweepArgs *__restrict__ args,
+                                                   const WorkItem *__restrict__ work, int nwork) {
+  int w;
+  if (!xcd_item(nwork, w)) return;
+  const int arg = __builtin_amdgcn_readfirstlane(work[w].arg);
+  const int bx = __builtin_amdgcn_readfirstlane(work[w].bx);
+  __shared__ R lds[PACKK_LDS];
+  k_packk_body<R, B0V>(batch_args(args, arg), bx, 0, 0, lds);
 }
 
 template <typename R, bool B0V>
@@ -1354,6 +1462,94 @@ __global__ __launch_bounds__(256) void k_sweepk_batch(const SweepArgs *__restric
   const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
   __shared__ R lds[SWEEPK_LDS];
   k_sweepk_body<R, B0V>(batch_args(args, arg), bx, by, bz, lds);
+}
+
+// The three sweeps of a small grid in one launch of one-wave blocks: the i and
+// the j march, the j sweep's velocity strip, the k tiles and the leftover k
+// columns.  Apart, each launch leaves most of the chip idle while a few waves
+// walk their two faces.  Parts start at multiples of NXCD and keep their own
+// XCD-aware order; the longest run first.  32^3 FP64: 0.017 + 0.016 + 0.013 +
+// 0.012 ms apart, 0.024 merged; 61x43x37 FP32-bulk 0.051 -> 0.027, 128x128x8
+// FP64 (k tiles packed) 0.101 -> 0.065.  A merged launch runs at the marches'
+// registers, one wave per SIMD in FP64 and two in FP32-bulk, which is why
+// larger grids keep the launches apart (default_shapes).
+enum { SP_MARCH_I = 0, SP_MARCH_J, SP_STRIP_J, SP_TILES, SP_KCOL, SP_COUNT };
+struct SweepPart {
+  void *F, *V;
+  int lo[3], hi[3], flo[3], fhi[3];
+  int nch, rp, gap;
+  int first, n;    // first block, blocks
+  int gx, gy;      // tiles along k and rows, of SP_TILES
+};
+struct SweepsArgs {
+  SweepArgs c;     // what the parts share
+  SweepPart p[SP_COUNT];
+};
+
+__device__ __forceinline__ SweepArgs sweep_args(const SweepsArgs &s, const SweepPart &p) {
+  SweepArgs a = s.c;
+  a.F = p.F;
+  a.V = p.V;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    a.lo[d] = p.lo[d];
+    a.hi[d] = p.hi[d];
+    a.flo[d] = p.flo[d];
+    a.fhi[d] = p.fhi[d];
+  }
+  a.nch = p.nch;
+  a.rp = p.rp;
+  a.gap = p.gap;
+  return a;
+}
+
+// block b of part p in the order its own launch would take
+__device__ __forceinline__ int part_block(const SweepPart &p, int b) {
+  const int per = (p.n + NXCD - 1) / NXCD;
+  b -= p.first;
+  const int L = (b % NXCD) * per + b / NXCD;
+  return L < p.n ? L : -1;
+}
+
+template <typename R, bool B0V, bool UT, bool ENT>
+__device__ __forceinline__ void k_sweeps_body(const SweepsArgs &s, const int b, R *lds) {
+  if (b < s.p[SP_MARCH_J].first) {
+    const SweepPart &p = s.p[SP_MARCH_I];
+    const int L = part_block(p, b), t = L / p.nch;
+    if (L >= 0) k_march_part<0, R, B0V, UT, ENT>(sweep_args(s, p), t >> 2, t & 3, L - t * p.nch);
+  } else if (b < s.p[SP_STRIP_J].first) {
+    const SweepPart &p = s.p[SP_MARCH_J];
+    const int L = part_block(p, b), t = L / p.nch;
+    if (L >= 0) k_march_part<1, R, B0V, UT, ENT>(sweep_args(s, p), t >> 2, t & 3, L - t * p.nch);
+  } else if (b < s.p[SP_TILES].first) {
+    const SweepPart &p = s.p[SP_STRIP_J];
+    const int L = part_block(p, b);
+    if (L >= 0) k_strip_part<1, R>(sweep_args(s, p), L >> 2, L & 3);
+  } else if (b < s.p[SP_KCOL].first) {
+    const SweepPart &p = s.p[SP_TILES];
+    const int L = part_block(p, b), t = L / p.gx;
+    if (L < 0) return;
+    if (p.rp > 1)
+      k_sweepk_pack<R, B0V, ENT>(sweep_args(s, p), L, lds);
+    else
+      k_sweepk_part<R, B0V, ENT>(sweep_args(s, p), L - t * p.gx, t % p.gy, t / p.gy, lds);
+  } else {
+    const SweepPart &p = s.p[SP_KCOL];
+    const int L = part_block(p, b);
+    if (L >= 0) k_kcol_part<R, B0V, ENT>(sweep_args(s, p), L, 0, 0, lds);
+  }
+}
+
+template <typename R, bool B0V, bool UT>
+__global__ __launch_bounds__(64)
+    __attribute__((amdgpu_waves_per_eu(MarchWaves<R>::n))) void k_sweeps(SweepsArgs s) {
+  static_assert(KCOL_LDS >= SWEEPK_LDS && KCOL_LDS >= PACKK_LDS, "LDS of the parts");
+  __shared__ R lds[KCOL_LDS];
+  if (halted(s.c.sc)) return;
+  if (carries_entropy(s.c.sc))
+    k_sweeps_body<R, B0V, UT, true>(s, blockIdx.x, lds);
+  else
+    k_sweeps_body<R, B0V, UT, false>(s, blockIdx.x, lds);
 }
 
 // Edge EMF from the edge velocities (va, vb), the two reconstructed face-B
@@ -1735,6 +1931,28 @@ __global__ __launch_bounds__(256)
     k_emf_march_body<0, R, false, B0V, UT>(a0, bx, by, bz);
   else
     k_emf_march_body<1, R, false, B0V, UT>(a1, bx, by, bz);
+}
+
+// The three edge fields of a small grid in one launch, one edge per thread (32^3
+// FP64: 0.035 ms apart, 0.0125 merged; 128x128x8 0.050 -> 0.033)
+struct EdgesArgs {
+  EmfArgs a[3];
+  int gx[3], n[3];  // blocks per (row, k) plane; blocks of direction D
+};
+
+template <typename R, bool B0V, bool UT>
+__global__ __launch_bounds__(256) void k_edges(EdgesArgs e, int total) {
+  int L;
+  if (!xcd_linear(total, L)) return;
+  const int r = L / 3, D = L - 3 * r;
+  if (r >= e.n[D]) return;
+  const int bz = r / e.gx[D], bx = r - bz * e.gx[D];
+  if (D == 0)
+    k_emf_march_body<0, R, false, B0V, UT>(e.a[0], bx, 0, bz);
+  else if (D == 1)
+    k_emf_march_body<1, R, false, B0V, UT>(e.a[1], bx, 0, bz);
+  else
+    k_emf_march_body<2, R, false, B0V, UT>(e.a[2], bx, 0, bz);
 }
 
 // staged form over whole 64-edge tiles along k (E_i, E_j): one wave per block
@@ -2270,8 +2488,16 @@ __global__ __launch_bounds__(256) void k_dt_batch(const DtArgs *__restrict__ arg
 // passes, because each later pass copies whole rows of the earlier ones, and
 // every source point is interior in all three axes, so no thread reads a
 // point another thread writes.
+//
+// In a step the launch also forms the cell-centred B of the same points, each
+// from its two faces at their sources, instead of a launch of its own that
+// reads the ghosts just written (256^3 FP64 0.091 + 0.033 -> 0.120 ms, FP32-bulk
+// 0.121 + 0.048 -> 0.155, 32^3 0.0165 -> 0.0134).
 struct GhostArgs {
   Grid g;
+  Geo geo;      // of the cell-centred B
+  double *M;    // cell-centred B of the points outside the active cells, or null
+  float *M32;   // its FP32 copy (FP32-bulk form), or null
   double *X;    // 6 cell fields, or null (not filled)
   double *B;    // 3 face fields, or null (not filled)
   float *X32;   // FP32 copies (FP32-bulk form), else null
@@ -2281,6 +2507,9 @@ struct GhostArgs {
 };
 
 __device__ __forceinline__ void globalize(GhostArgs &a) {
+  globalize(a.geo);
+  gptr(a.M);
+  gptr(a.M32);
   gptr(a.X);
   gptr(a.B);
   gptr(a.X32);
@@ -2336,12 +2565,9 @@ __device__ __forceinline__ int pole_k(const Grid &g, int k) {
 // The points of the box outside the active cells, walked as three slabs:
 // i outside [s0, e0] (all j, k), then j outside [s1, e1] (i active, all k),
 // then k outside [s2, e2] (i, j active); k fastest in each, 256 per block.
-// The box is N - shrink points per axis (shrink 1 leaves out the upper face
-// slot, for cell quantities formed from both faces of a cell).
-__device__ __forceinline__ bool ghost_point(const Grid &g, int bx, int &i, int &j, int &k,
-                                           int shrink = 0) {
+__device__ __forceinline__ bool ghost_point(const Grid &g, int bx, int &i, int &j, int &k) {
   const int n0 = g.e[0] - g.s[0] + 1, n1 = g.e[1] - g.s[1] + 1, n2 = g.e[2] - g.s[2] + 1;
-  const int N0 = g.N[0] - shrink, N1 = g.N[1] - shrink, N2 = g.N[2] - shrink;
+  const int N0 = g.N[0], N1 = g.N[1], N2 = g.N[2];
   long p = (long)bx * 256 + threadIdx.y * 64 + threadIdx.x;
   const long ca = (long)(N0 - n0) * N1 * N2, cb = (long)n0 * (N1 - n1) * N2;
   const long cc = (long)n0 * n1 * (N2 - n2);
@@ -2374,6 +2600,39 @@ __device__ __forceinline__ bool ghost_point(const Grid &g, int bx, int &i, int &
   return false;
 }
 
+// Where face f of field B at point x comes from: its offset (its own where no
+// map moves it), whether it changes sign (pole) and whether it is 0 (fixed)
+template <int f>
+__device__ __forceinline__ long ghost_face(const GhostArgs &a, const int x[3], bool &neg,
+                                           bool &zero) {
+  const Grid &g = a.g;
+  int m[3];
+  zero = false;
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    m[d] = gmap(x[d], g.s[d], g.e[d], a.bc[1][2 * d], a.bc[1][2 * d + 1], d == f ? 1 : 0);
+    zero = zero || fixed_ghost(x[d], g.s[d], g.e[d], a.bc[1][2 * d], a.bc[1][2 * d + 1],
+                               d == f ? 1 : 0);
+  }
+  neg = pole_row(g, x[1], a.bc[1][2], a.bc[1][3], f == 1 ? 1 : 0);
+  if (neg) m[2] = pole_k(g, x[2]);
+  if (f == 0) neg = false;
+  return m[0] * g.st[0] + m[1] * g.st[1] + m[2];
+}
+
+// Cell-centred B component f of a point outside the active cells, from its two
+// faces at their sources: the lower one's value is given, the upper one may be
+// an active face or another ghost
+template <int f>
+__device__ __forceinline__ double ghost_cell_b(const GhostArgs &a, const int x[3], double lower) {
+  int y[3] = {x[0], x[1], x[2]};
+  y[f] += 1;
+  bool neg, zero;
+  const long s = ghost_face<f>(a, y, neg, zero);
+  const double b = a.B[f * a.g.fs + s];
+  return cell_b_of(lower, zero ? 0.0 : (neg ? -b : b), a.geo, x[f], f);
+}
+
 __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, const int by,
                                         const int bz) {
   if (halted(a.sc)) return;
@@ -2401,21 +2660,10 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
                   gmap(j, g.s[1], g.e[1], a.bc[0][2], a.bc[0][3], 0) * g.st[1] +
                   (px ? pole_k(g, k) : gmap(k, g.s[2], g.e[2], a.bc[0][4], a.bc[0][5], 0));
   long sb[3];
-  bool pb[3], fb[3];
-#pragma unroll
-  for (int f = 0; f < 3; f++) {
-    int m[3];
-    fb[f] = false;  // in a fixed ghost slab of this face field: 0
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-      m[d] = gmap(x[d], g.s[d], g.e[d], a.bc[1][2 * d], a.bc[1][2 * d + 1], d == f ? 1 : 0);
-      fb[f] = fb[f] || fixed_ghost(x[d], g.s[d], g.e[d], a.bc[1][2 * d], a.bc[1][2 * d + 1],
-                                   d == f ? 1 : 0);
-    }
-    pb[f] = pole_row(g, j, a.bc[1][2], a.bc[1][3], f == 1 ? 1 : 0);
-    if (pb[f]) m[2] = pole_k(g, k);
-    sb[f] = m[0] * g.st[0] + m[1] * g.st[1] + m[2];
-  }
+  bool neg[3], fb[3];
+  sb[0] = ghost_face<0>(a, x, neg[0], fb[0]);
+  sb[1] = ghost_face<1>(a, x, neg[1], fb[1]);
+  sb[2] = ghost_face<2>(a, x, neg[2], fb[2]);
   // p_S moves only while the step carries it, or where this step's cell update
   // has just written one that is not 0 (everything outside a step)
   const int nx = !a.sc || a.sc->ent || a.sc->ent_next ? 6 : 5;
@@ -2449,11 +2697,22 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
   }
 #pragma unroll
   for (int f = 0; f < 3; f++) {
-    if (sb[f] != c) {
-      const bool neg = pb[f] && f != 0;
-      if (a.B) bv[f] = neg ? -a.B[f * g.fs + sb[f]] : a.B[f * g.fs + sb[f]];
-      if (a.B32) bw[f] = neg ? -a.B32[f * g.fs + sb[f]] : a.B32[f * g.fs + sb[f]];
+    if (a.B) {
+      const double b = a.B[f * g.fs + sb[f]];
+      bv[f] = fb[f] ? 0.0 : (neg[f] ? -b : b);
     }
+    if (a.B32) {
+      const float b = a.B32[f * g.fs + sb[f]];
+      bw[f] = fb[f] ? 0.0f : (neg[f] ? -b : b);
+    }
+  }
+  // the cell-centred B of the same point (the box without the upper face slot)
+  const bool mags = (a.M || a.M32) && i < g.N[0] - 1 && j < g.N[1] - 1 && k < g.N[2] - 1;
+  double mb[3];
+  if (mags) {
+    mb[0] = ghost_cell_b<0>(a, x, bv[0]);
+    mb[1] = ghost_cell_b<1>(a, x, bv[1]);
+    mb[2] = ghost_cell_b<2>(a, x, bv[2]);
   }
   if (fx) {  // fixed: the constants replace rho, v, p; p_S as mapped
     const double fixv[5] = {1.0, 0.0, 0.0, 0.0, 1.0};
@@ -2478,13 +2737,13 @@ __device__ __forceinline__ void k_ghost_body(const GhostArgs &a, const int bx, c
   }
 #pragma unroll
   for (int f = 0; f < 3; f++) {
-    if (fb[f]) {
-      bv[f] = 0.0;
-      bw[f] = 0.0f;
-    }
     if (sb[f] != c || fb[f]) {
       if (a.B) a.B[f * g.fs + c] = bv[f];
       if (a.B32) a.B32[f * g.fs + c] = bw[f];
+    }
+    if (mags) {
+      if (a.M) a.M[f * g.fs + c] = mb[f];
+      if (a.M32) a.M32[f * g.fs + c] = (float)mb[f];
     }
   }
 }
@@ -2514,33 +2773,14 @@ struct MagsArgs {
   Grid g;
   Geo geo;
   const double *B;
-  double *M;   // or null (not written)
-  float *M32;  // FP32 copy (FP32-bulk form), else null
-  const Scal *sc;  // run control of a step's launch (null outside a step)
+  double *M;
 };
 
-__device__ __forceinline__ void globalize(MagsArgs &a) {
-  globalize(a.geo);
-  gptr(a.B);
-  gptr(a.M);
-  gptr(a.M32);
-  gptr(a.sc);
-}
-
-template <bool SHELL = false>
-__device__ __forceinline__ void k_mags_body(const MagsArgs &a, const int bx, const int by,
-                                       const int bz) {
-  if (halted(a.sc)) return;
+__device__ __forceinline__ void k_mags_body(const MagsArgs &a, const int bx, const int bz) {
   const Grid &g = a.g;
-  (void)by;
-  int i, j, k;
-  if (SHELL) {  // only the points outside the active cells (the cell update forms the rest)
-    (void)bz;
-    if (!ghost_point(g, bx, i, j, k, 1)) return;
-  } else {
-    if (!row_point(0, g.N[2] - 2, 0, g.N[1] - 2, bx, k, j)) return;
-    i = bz;
-  }
+  int j, k;
+  if (!row_point(0, g.N[2] - 2, 0, g.N[1] - 2, bx, k, j)) return;
+  const int i = bz;
   const long c = i * g.st[0] + j * g.st[1] + k;
   const int idx[3] = {i, j, k};
   // all three components before the first store (a load after a store
@@ -2549,10 +2789,7 @@ __device__ __forceinline__ void k_mags_body(const MagsArgs &a, const int bx, con
 #pragma unroll
   for (int m = 0; m < 3; m++) b[m] = cell_b(a.B + m * g.fs, a.geo, c, g.st[m], idx[m], m);
 #pragma unroll
-  for (int m = 0; m < 3; m++) {
-    if (a.M) a.M[m * g.fs + c] = b[m];
-    if (a.M32) a.M32[m * g.fs + c] = (float)b[m];
-  }
+  for (int m = 0; m < 3; m++) a.M[m * g.fs + c] = b[m];
 }
 
 // Whether a state needs the entropy channel (carries_entropy): p_S not 0
@@ -2601,32 +2838,10 @@ __global__ __launch_bounds__(256) void k_to32(const double *__restrict__ src,
 }
 
 __global__ __launch_bounds__(256) void k_mags(MagsArgs a, int gx, int gy, int gz) {
-  int bx, by, bz;
+  int bx, bz;
   (void)gy;
-  by = 0;
   if (!xcd_patch(gx, gz, bx, bz)) return;
-  k_mags_body(a, bx, by, bz);
-}
-
-// cell-centred B of the points outside the active cells (a step's cell
-// update writes the active ones)
-__global__ __launch_bounds__(256) void k_mags_shell(MagsArgs a, int gx, int gy, int gz) {
-  int bx, by, bz;
-  if (!xcd_block<false>(gx, gy, gz, bx, by, bz)) return;
-  k_mags_body<true>(a, bx, by, bz);
-}
-
-// one launch for many grids: block w runs work-list entry w (argument set, block)
-__global__ __launch_bounds__(256) void k_mags_batch(const MagsArgs *__restrict__ args,
-                                                    const WorkItem *__restrict__ work, int nwork) {
-  int w;
-  if (!xcd_item(nwork, w)) return;
-  // uniform per block: keep the argument set in scalar registers
-  const int arg = __builtin_amdgcn_readfirstlane(work[w].arg);
-  const int bx = __builtin_amdgcn_readfirstlane(work[w].bx);
-  const int by = __builtin_amdgcn_readfirstlane(work[w].by);
-  const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
-  k_mags_body<true>(batch_args(args, arg), bx, by, bz);
+  k_mags_body(a, bx, bz);
 }
 
 // ---------------------------------------------------------------------------
@@ -3126,6 +3341,9 @@ struct gk_solver {
   int chunk;           // faces per thread in the marching sweeps
   int emf_chunk;       // edges per thread in the marching EMF kernels
   int emf_stage;       // bit D: E_D (D = 0, 1) over whole 64-edge k tiles staged in LDS
+  int merge_sweeps;    // alone: all sweeps in one launch (k_sweeps)
+  int merge_edges;     // alone: all edge fields in one launch, one edge per thread (k_edges)
+  int merge_chunk;     // faces per thread in the marches of a merged launch
   double rho_floor, p_floor;  // positivity floors
   double grav[3];      // uniform gravity
   struct gk_batch *batch;  // batch that owns the stepping, if any
@@ -3293,6 +3511,16 @@ static hipError_t upload(gk_solver *s, void *dst, const void *src, size_t bytes)
 // (8, 4) in FP32-bulk within 3%; 256^3 (32, 16) best.  The pair that was the
 // default for every size, (32, 16), had cost 32^3 3.8x and 128x128x8 2.3x.
 // gk_autotune times the candidates on the grid itself.
+//
+// Small grids stepped alone take all sweeps in one launch (k_sweeps) up to
+// 6e5 cells in FP64 and 1e6 in FP32-bulk, and all edge fields in one
+// (k_edges) up to 3e5 (ms per step with the launches apart / merged: 32^3
+// FP64 0.105 / 0.060; 48^3 0.143 / 0.108; 128x128x8 0.180 / 0.140; 64^3 0.208
+// / 0.175; 96x72x60 0.329 / 0.300; 96^3 0.509 / 0.530; FP32-bulk 64^3 0.146 /
+// 0.116, 80^3 0.283 / 0.232, 96^3 0.309 / 0.297; edges alone 64^3 0.194 /
+// 0.175, 96x72x60 0.086 / 0.088 ms).  Merged marches share the chip, so they
+// may be longer than a march that has it alone: 2 faces per thread best at
+// 32^3, 4 at 61x43x37, 8 at 48^3, 12 at 128x128x8 and above.
 static void default_shapes(gk_solver *s) {
   const double n = (double)s->ni * s->nj * s->nk;
   if (n >= 1.2e7) {
@@ -3315,6 +3543,9 @@ static void default_shapes(gk_solver *s) {
     s->chunk = 2;
     s->emf_chunk = 2;
   }
+  s->merge_sweeps = n < (s->precision == 1 ? 1e6 : 6e5);
+  s->merge_edges = n < 3e5;
+  s->merge_chunk = n < 5e4 ? 2 : n < 1e5 ? 4 : n < 1.25e5 ? 8 : 12;
 }
 
 extern "C" int gk_create(const gk_grid_desc *d, gk_solver **out) {
@@ -3720,17 +3951,6 @@ static int patch_blocks(const dim3 &g) {
   return (int)((g.x + PATCH - 1) / PATCH * PATCH * ((g.z + PATCH - 1) / PATCH) * PATCH);
 }
 
-// cell-centred B of the points outside the active cells, in the box minus
-// the upper face slot
-static dim3 mags_shell_grid(const Grid &g) {
-  long n = 1, t = 1;
-  for (int d = 0; d < 3; d++) {
-    n *= g.e[d] - g.s[d] + 1;
-    t *= g.N[d] - 1;
-  }
-  return dim3((unsigned)((t - n + 255) / 256), 1, 1);
-}
-
 // cell-centred B over the box minus the upper face slot
 static dim3 mags_grid(const Grid &g) {
   return dim3(row_blocks(0, g.N[2] - 2, 0, g.N[1] - 2), 1, g.N[0] - 1);
@@ -3738,6 +3958,7 @@ static dim3 mags_grid(const Grid &g) {
 
 static void launch_ghost(gk_solver *s, double *X, double *B) {
   GhostArgs a;
+  memset(&a, 0, sizeof a);
   a.g = s->g;
   a.X = X;
   a.B = B;
@@ -3756,8 +3977,6 @@ static void launch_mags(gk_solver *s, const double *B, double *M) {
   a.geo = s->geo;
   a.B = B;
   a.M = M;
-  a.M32 = nullptr;
-  a.sc = nullptr;
   const dim3 gr = mags_grid(s->g);
   const int tot = patch_blocks(gr);
   k_mags<<<dim3((tot + NXCD - 1) / NXCD * NXCD), dim3(64, 4), 0, s->stream>>>(a, gr.x, gr.y, gr.z);
@@ -3950,23 +4169,29 @@ void resolve_timers(gk_solver *s) {
 // Ids follow the order a step runs them in: a batch launches its stages in
 // id order (the k_pole_* and k_ring_* stages exist on pole ring-averaged grids)
 enum StageKernel {
-  SK_BEGIN = 0, SK_SWEEP_I, SK_VSTRIP_I, SK_SWEEP_J, SK_VSTRIP_J, SK_SWEEP_K, SK_KREM, SK_EMF_I, SK_EMF_J,
+  SK_BEGIN = 0, SK_SWEEP_I, SK_VSTRIP_I, SK_SWEEP_J, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_I, SK_EMF_J,
   SK_EMF_K, SK_EMF_IS, SK_EMF_JS, SK_POLE_E, SK_CT, SK_POLE_B, SK_CELL, SK_RING_ROWS,
-  SK_RING_CURL, SK_RING_FIX, SK_RING_MAGS, SK_GHOST, SK_MAGS, SK_RING_DT, SK_COUNT
+  SK_RING_CURL, SK_RING_FIX, SK_RING_MAGS, SK_GHOST, SK_RING_DT, SK_COUNT,
+  // stages of a small grid stepped alone (never in a batch): all sweeps and
+  // all edge fields in one launch each, timed under the first stage's name
+  SK_SWEEPS = SK_COUNT, SK_EDGES, SK_ALL
 };
-static const char *const sk_name[SK_COUNT] = {
-    "k_begin", "k_sweep_i", "k_vstrip_i", "k_sweep_j", "k_vstrip_j", "k_sweep_k", "k_krem_k", "k_emf_i",
+static const char *const sk_name[SK_ALL] = {
+    "k_begin", "k_sweep_i", "k_vstrip_i", "k_sweep_j", "k_vstrip_j", "k_sweep_k", "k_sweep_k", "k_krem_k", "k_emf_i",
     "k_emf_j", "k_emf_k", "k_emf_i_tiles", "k_emf_j_tiles", "k_pole_e", "k_ct", "k_pole_b",
-    "k_cell", "k_ring_rows", "k_ring_curl", "k_ring_fix", "k_ring_mags", "k_ghost", "k_mags",
-    "k_ring_dt"};
+    "k_cell", "k_ring_rows", "k_ring_curl", "k_ring_fix", "k_ring_mags", "k_ghost",
+    "k_ring_dt", "k_sweep_i", "k_emf_i"};
+
+static_assert(sizeof(SweepsArgs) + 64 <= 4096 && sizeof(EdgesArgs) + 64 <= 4096, "kernel arguments");
 
 union StageArgs {
+  SweepsArgs sa;
+  EdgesArgs ed;
   SweepArgs sw;
   EmfArgs em;
   CtArgs ct;
   CellArgs ce;
   GhostArgs gh;
-  MagsArgs mg;
   RingArgs rg;
   DtArgs dt;
   Scal *sc;
@@ -3976,7 +4201,7 @@ static size_t stage_arg_size(int kid) {
   switch (kid) {
     case SK_BEGIN: return sizeof(Scal *);
     case SK_SWEEP_I: case SK_VSTRIP_I: case SK_SWEEP_J: case SK_VSTRIP_J: case SK_SWEEP_K:
-    case SK_KREM:
+    case SK_PACK_K: case SK_KREM:
       return sizeof(SweepArgs);
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return sizeof(EmfArgs);
@@ -3987,7 +4212,7 @@ static size_t stage_arg_size(int kid) {
     case SK_POLE_E: case SK_POLE_B: case SK_RING_ROWS: case SK_RING_CURL: case SK_RING_FIX:
     case SK_RING_MAGS:
       return sizeof(RingArgs);
-    default: return sizeof(MagsArgs);
+    default: return 0;
   }
 }
 
@@ -3995,7 +4220,7 @@ static const void *stage_arg_ptr(int kid, const StageArgs &u) {
   switch (kid) {
     case SK_BEGIN: return &u.sc;
     case SK_SWEEP_I: case SK_VSTRIP_I: case SK_SWEEP_J: case SK_VSTRIP_J: case SK_SWEEP_K:
-    case SK_KREM:
+    case SK_PACK_K: case SK_KREM:
       return &u.sw;
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return &u.em;
@@ -4006,7 +4231,7 @@ static const void *stage_arg_ptr(int kid, const StageArgs &u) {
     case SK_POLE_E: case SK_POLE_B: case SK_RING_ROWS: case SK_RING_CURL: case SK_RING_FIX:
     case SK_RING_MAGS:
       return &u.rg;
-    default: return &u.mg;
+    default: return nullptr;
   }
 }
 
@@ -4030,6 +4255,49 @@ static int point_blocks(const SweepArgs &v) {
   return (int)((n + 255) / 256);
 }
 
+// The sweeps' launches (all after k_begin) as the parts of one k_sweeps launch
+static void merge_sweeps(std::vector<Launch> &out) {
+  Launch M;
+  memset(&M, 0, sizeof M);
+  SweepsArgs &s = M.u.sa;
+  M.kid = SK_SWEEPS;
+  s.c = out[1].u.sw;
+  const Launch *part[SP_COUNT] = {};
+  for (size_t q = 1; q < out.size(); q++) switch (out[q].kid) {
+      case SK_SWEEP_I: part[SP_MARCH_I] = &out[q]; break;
+      case SK_SWEEP_J: part[SP_MARCH_J] = &out[q]; break;
+      case SK_VSTRIP_J: part[SP_STRIP_J] = &out[q]; break;
+      case SK_SWEEP_K: case SK_PACK_K: part[SP_TILES] = &out[q]; break;
+      case SK_KREM: part[SP_KCOL] = &out[q]; break;
+    }
+  int first = 0;
+  for (int q = 0; q < SP_COUNT; q++) {
+    SweepPart &p = s.p[q];
+    p.first = first;
+    p.gx = p.gy = 1;
+    if (!part[q]) continue;
+    const SweepArgs &a = part[q]->u.sw;
+    const dim3 g = part[q]->grid;
+    p.F = a.F;
+    p.V = a.V;
+    memcpy(p.lo, a.lo, sizeof p.lo);
+    memcpy(p.hi, a.hi, sizeof p.hi);
+    memcpy(p.flo, a.flo, sizeof p.flo);
+    memcpy(p.fhi, a.fhi, sizeof p.fhi);
+    p.nch = a.nch;
+    p.rp = a.rp;
+    p.gap = a.gap;
+    // blocks of 256 points are four one-wave blocks here
+    p.n = (int)(g.x * g.y * g.z) * (q <= SP_STRIP_J ? 4 : 1);
+    p.gx = (int)g.x;
+    p.gy = (int)g.y;
+    first += (p.n + NXCD - 1) / NXCD * NXCD;
+  }
+  M.grid = dim3(first, 1, 1);
+  out.resize(1);
+  out.push_back(M);
+}
+
 static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out) {
   out.clear();
   const Grid &g = s->g;
@@ -4039,7 +4307,8 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
   const double *Mm1 = s->M[r.b_m1], *M = s->M[r.b_0];
   double *Bn = s->B[r.b_n], *Mn = s->M[r.b_n];
   double *Xn = s->X[1 - r.cur];
-  const int ch = s->chunk;
+  const bool merge = s->merge_sweeps && !s->batch, direct = s->merge_edges && !s->batch;
+  const int ch = merge ? s->merge_chunk : s->chunk;
   // the stencil kernels read the state in their compute type
   const bool f32 = s->precision == 1;
   const void *Xs = f32 ? (const void *)s->X32[r.cur] : (const void *)X;
@@ -4055,6 +4324,7 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
   L.u.sc = s->sc;
   out.push_back(L);
 
+  EdgesArgs ed;
   // directional sweeps: face fluxes + face velocities
   for (int D = 0; D < 3; D++) {
     SweepArgs a;
@@ -4093,6 +4363,7 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
     // (256^3 at the default of 64: 128-129 faces per thread, 2 chunks of
     // 1024 waves each); smaller grids stepped alone keep the parallelism
     auto long_march = [&](SweepArgs &m, int cols) {
+      if (merge) return false;
       const int n2 = march_chunks(m.hi[D] - m.lo[D] + 1, std::min(2 * ch, 4096));
       if ((long)cols * n2 < 1024L * 64 * (f32 ? 2 : 1)) return false;
       m.nch = n2;
@@ -4158,10 +4429,15 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
       const int wk = a.hi[2] - a.lo[2] + 1;
       const int rem = wk % 64;
       SweepArgs m = a;
+      m.rp = wk <= 32 ? std::min(64 / wk, PACKSPAN / (wk + 7)) : 1;
       const bool split = wk >= 64 && rem > 0 && rem < 32;
       if (split) m.hi[2] = a.hi[2] - rem;
       L.kid = SK_SWEEP_K;
       L.grid = dim3((m.hi[2] - m.lo[2] + 64) / 64, m.hi[1] - m.lo[1] + 1, m.hi[0] - m.lo[0] + 1);
+      if (m.rp > 1) {
+        L.kid = SK_PACK_K;
+        L.grid = dim3((L.grid.y * L.grid.z + m.rp - 1) / m.rp, 1, 1);
+      }
       L.u.sw = m;
       out.push_back(L);
       if (split) {
@@ -4175,6 +4451,7 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
       }
     }
   }
+  if (merge) merge_sweeps(out);
   // edge electric fields
   for (int D = 0; D < 3; D++) {
     EmfArgs a;
@@ -4197,6 +4474,13 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
       a.hi[d] = Ee[d] + (d == D ? 0 : 1);
     }
     const int MA = D == 1 ? 0 : 1, RA = D == 1 ? 1 : 0;
+    if (direct) {
+      a.nch = a.hi[MA] - a.lo[MA] + 1;
+      ed.a[D] = a;
+      ed.gx[D] = row_blocks(a.lo[2], a.hi[2], a.lo[RA], a.hi[RA]);
+      ed.n[D] = ed.gx[D] * a.nch;
+      continue;
+    }
     a.nch = march_chunks(a.hi[MA] - a.lo[MA] + 1, s->emf_chunk);
     const int nf = a.nch;
     // staged E_i / E_j (bit D of emf_stage; by default both in FP64, E_j in
@@ -4223,6 +4507,12 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
       out.push_back(L);
       L.rest = false;
     }
+  }
+  if (direct) {
+    L.kid = SK_EDGES;
+    L.grid = dim3(3 * std::max(ed.n[0], std::max(ed.n[1], ed.n[2])), 1, 1);
+    L.u.ed = ed;
+    out.push_back(L);
   }
   // pole ring averaging: arguments shared by its kernels
   RingArgs ra;
@@ -4342,24 +4632,15 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
     a.X32 = f32 ? s->X32[1 - r.cur] : nullptr;
     a.B32 = f32 ? s->B32[r.b_n] : nullptr;
     memcpy(a.bc, s->bc, sizeof(a.bc));
+    // with the cell-centred B of the same points (FP32-bulk: only the FP32 copy
+    // is read)
+    a.geo = s->geo;
+    a.M = f32 ? nullptr : Mn;
+    a.M32 = f32 ? s->M32[r.b_n] : nullptr;
     a.sc = s->sc;
     L.kid = SK_GHOST;
     L.grid = ghost_grid(g);
     L.u.gh = a;
-    out.push_back(L);
-  }
-  {
-    MagsArgs a;
-    memset(&a, 0, sizeof a);
-    a.g = g;
-    a.geo = s->geo;
-    a.B = Bn;
-    a.M = f32 ? nullptr : Mn;  // FP32-bulk: only the FP32 copy is read
-    a.M32 = f32 ? s->M32[r.b_n] : nullptr;
-    a.sc = s->sc;
-    L.kid = SK_MAGS;  // ghost cells only (k_mags_shell)
-    L.grid = mags_shell_grid(g);
-    L.u.mg = a;
     out.push_back(L);
   }
   if (s->ring) {
@@ -4401,10 +4682,11 @@ static void launch_one(const Launch &L, hipStream_t st) {
   switch (L.kid) {
     case SK_BEGIN: k_begin<<<1, NSLOT, 0, st>>>(L.u.sc); break;
     case SK_SWEEP_I: k_march<0, R, B0V, UT><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
-    case SK_VSTRIP_I: k_sweep<0, R, B0V><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
+    case SK_VSTRIP_I: k_sweep<0, R><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
     case SK_SWEEP_J: k_march<1, R, B0V, UT><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
-    case SK_VSTRIP_J: k_sweep<1, R, B0V><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
+    case SK_VSTRIP_J: k_sweep<1, R><<<g1, blk, 0, st>>>(L.u.sw, gx, gy, gz); break;
     case SK_SWEEP_K: k_sweepk<R, B0V><<<g1, dim3(64), 0, st>>>(L.u.sw, gx, gy, gz); break;
+    case SK_PACK_K: k_packk<R, B0V><<<g1, dim3(64), 0, st>>>(L.u.sw, gx, gy, gz); break;
     case SK_KREM: k_kcol<R, B0V><<<g1, dim3(64), 0, st>>>(L.u.sw, gx, gy, gz); break;
     case SK_EMF_I: k_emf_march<0, R, B0V, UT><<<g1, blk, 0, st>>>(L.u.em, gx, gy, gz); break;
     case SK_EMF_J: k_emf_march<1, R, B0V, UT><<<g1, blk, 0, st>>>(L.u.em, gx, gy, gz); break;
@@ -4414,7 +4696,6 @@ static void launch_one(const Launch &L, hipStream_t st) {
     case SK_CT: k_ct<R><<<g1, blk, 0, st>>>(L.u.ct, gx, gy, gz); break;
     case SK_CELL: k_cell<R, B0V><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
     case SK_GHOST: k_ghost<<<g1, blk, 0, st>>>(L.u.gh, gx, gy, gz); break;
-    case SK_MAGS: k_mags_shell<<<g1, blk, 0, st>>>(L.u.mg, gx, gy, gz); break;
     case SK_POLE_E: k_pole_e<R><<<L.grid, dim3(64), 0, st>>>(L.u.rg); break;
     case SK_POLE_B: k_pole_b<<<L.grid, dim3(256), 0, st>>>(L.u.rg); break;
     case SK_RING_ROWS: k_ring_rows<R><<<L.grid, dim3(64), 0, st>>>(L.u.rg); break;
@@ -4422,6 +4703,8 @@ static void launch_one(const Launch &L, hipStream_t st) {
     case SK_RING_FIX: k_ring_fix<<<L.grid, dim3(64), 0, st>>>(L.u.rg); break;
     case SK_RING_MAGS: k_ring_mags<<<L.grid, dim3(256), 0, st>>>(L.u.rg); break;
     case SK_RING_DT: k_dt<B0V><<<L.grid, dim3(64, 4), 0, st>>>(L.u.dt); break;
+    case SK_SWEEPS: k_sweeps<R, B0V, UT><<<gx, dim3(64), 0, st>>>(L.u.sa); break;
+    case SK_EDGES: k_edges<R, B0V, UT><<<g1, blk, 0, st>>>(L.u.ed, total); break;
   }
 }
 
@@ -4432,10 +4715,11 @@ static void launch_batch(int kid, const void *args, const WorkItem *work, int nw
   switch (kid) {
     case SK_BEGIN: k_begin_batch<<<nwork, NSLOT, 0, st>>>((Scal *const *)args, nwork); break;
     case SK_SWEEP_I: k_march_batch<0, R, B0V, UT><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
-    case SK_VSTRIP_I: k_sweep_batch<0, R, B0V><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
+    case SK_VSTRIP_I: k_sweep_batch<0, R><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
     case SK_SWEEP_J: k_march_batch<1, R, B0V, UT><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
-    case SK_VSTRIP_J: k_sweep_batch<1, R, B0V><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
+    case SK_VSTRIP_J: k_sweep_batch<1, R><<<nblocks, blk, 0, st>>>((const SweepArgs *)args, work, nwork); break;
     case SK_SWEEP_K: k_sweepk_batch<R, B0V><<<nblocks, dim3(64), 0, st>>>((const SweepArgs *)args, work, nwork); break;
+    case SK_PACK_K: k_packk_batch<R, B0V><<<nblocks, dim3(64), 0, st>>>((const SweepArgs *)args, work, nwork); break;
     case SK_KREM: k_kcol_batch<R, B0V><<<nblocks, dim3(64), 0, st>>>((const SweepArgs *)args, work, nwork); break;
     case SK_EMF_I: k_emf_march_batch<0, R, B0V, UT><<<nblocks, blk, 0, st>>>((const EmfArgs *)args, work, nwork); break;
     case SK_EMF_J: k_emf_march_batch<1, R, B0V, UT><<<nblocks, blk, 0, st>>>((const EmfArgs *)args, work, nwork); break;
@@ -4445,7 +4729,6 @@ static void launch_batch(int kid, const void *args, const WorkItem *work, int nw
     case SK_CT: k_ct_batch<R><<<nblocks, blk, 0, st>>>((const CtArgs *)args, work, nwork); break;
     case SK_CELL: k_cell_batch<R, B0V><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
     case SK_GHOST: k_ghost_batch<<<nblocks, blk, 0, st>>>((const GhostArgs *)args, work, nwork); break;
-    case SK_MAGS: k_mags_batch<<<nblocks, blk, 0, st>>>((const MagsArgs *)args, work, nwork); break;
     case SK_POLE_E: k_pole_e_batch<R><<<nblocks, dim3(64), 0, st>>>((const RingArgs *)args, work, nwork); break;
     case SK_POLE_B: k_pole_b_batch<<<nblocks, dim3(256), 0, st>>>((const RingArgs *)args, work, nwork); break;
     case SK_RING_ROWS: k_ring_rows_batch<R><<<nblocks, dim3(64), 0, st>>>((const RingArgs *)args, work, nwork); break;
@@ -4876,15 +5159,18 @@ extern "C" int gk_set_tuning(gk_solver *s, int param, int value) {
   if (param == GK_TUNE_EMF_STAGE) {
     if (value < 0 || value > 3) return GK_ERR_ARG;
     s->emf_stage = value;
+    s->merge_edges = 0;  // a length or form asked for is the one that runs
     return GK_OK;
   }
   if (value < 1 || value > 4096) return GK_ERR_ARG;
   if (param == GK_TUNE_CHUNK) {
     s->chunk = value;
+    s->merge_sweeps = 0;
     return GK_OK;
   }
   if (param == GK_TUNE_EMF_CHUNK) {
     s->emf_chunk = value;
+    s->merge_edges = 0;
     return GK_OK;
   }
   return GK_ERR_ARG;
@@ -4984,7 +5270,7 @@ static void solo_order(int kid, dim3 gr, int idx, std::vector<WorkItem> &out) {
     case SK_CT: case SK_CELL:
       mode = gy == 1 ? 2 : 0;
       break;
-    default:  // SK_VSTRIP_I, SK_VSTRIP_J, SK_SWEEP_K, SK_KREM, SK_EMF_K, SK_MAGS, the ring stages
+    default:  // SK_VSTRIP_I, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_K, the ring stages
       mode = 0;
   }
   if (mode == 2) {
@@ -5394,7 +5680,7 @@ struct TuneKey {
   }
 };
 struct TunePick {
-  int chunk, emf_chunk, emf_stage;
+  int chunk, emf_chunk, emf_stage, merge_sweeps, merge_edges;
 };
 static std::vector<std::pair<TuneKey, TunePick>> g_tune_cache;
 
@@ -5407,6 +5693,8 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
       s->chunk = e.second.chunk;
       s->emf_chunk = e.second.emf_chunk;
       s->emf_stage = e.second.emf_stage;
+      s->merge_sweeps = e.second.merge_sweeps;
+      s->merge_edges = e.second.merge_edges;
       if (best) *best = e.second.chunk;
       return GK_OK;
     }
@@ -5486,6 +5774,13 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
   const int cand_e[] = {2, 4, 8, 16, 32};
   int pick = s->chunk, pick_e = s->emf_chunk, pick_s = s->emf_stage;
   float best_ms = 1e30f;
+  // merged launches, where the grid has them, against the best march apart (the
+  // march lengths are also what the grid takes inside a batch, which does not
+  // merge)
+  int merge_s = s->merge_sweeps, merge_e = s->merge_edges;
+  float ms_s = 1e30f, ms_e = 1e30f;
+  if (rc == GK_OK && merge_s) rc = trial(ms_s);
+  s->merge_sweeps = 0;
   for (int c : cand) {
     if (rc != GK_OK) break;
     if (c > 2 * maxlen && c != cand[0]) break;
@@ -5498,6 +5793,10 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
     }
   }
   s->chunk = pick;
+  merge_s = ms_s < best_ms;
+  s->merge_sweeps = merge_s;
+  if (rc == GK_OK && merge_e) rc = trial(ms_e);
+  s->merge_edges = 0;
   best_ms = 1e30f;
   for (int c : cand_e) {
     if (rc != GK_OK) break;
@@ -5528,16 +5827,19 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
       }
     }
   }
+  merge_e = ms_e < best_ms;
   s->timing = keep_timing;
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   (void)hipFreeAsync(save, s->stream);
   (void)hipStreamSynchronize(s->stream);
+  s->merge_sweeps = merge_s;
+  s->merge_edges = merge_e;
   if (rc != GK_OK) return rc;
   s->chunk = pick;
   s->emf_chunk = pick_e;
   s->emf_stage = pick_s;
-  g_tune_cache.push_back({key, TunePick{pick, pick_e, pick_s}});
+  g_tune_cache.push_back({key, TunePick{pick, pick_e, pick_s, merge_s, merge_e}});
   if (best) *best = pick;
   return GK_OK;
 }
