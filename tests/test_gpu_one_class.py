@@ -43,8 +43,8 @@ def test_one_class_steps_like_all_classes(kind, n):
             rows = rows.reshape(n_a, c, STRIDE).astype(np.float32)
             assert (rows == rows[:, :1]).all()
             off += rows.size * 8
-        prim = [np.ascontiguousarray(P.gas(f)) for f in range(6)]
-        bface = [np.ascontiguousarray(P.gem(f)) for f in range(3)]
+        prim = [np.array(P.gas(f)) for f in range(6)]
+        bface = [np.array(P.gem(f)) for f in range(3)]
     finally:
         P.close()
     apart = bytearray(blob)
