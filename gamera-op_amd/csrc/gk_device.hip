@@ -1196,7 +1196,6 @@ constexpr int KSPAN = 72;
 constexpr int PACKSPAN = 112;
 constexpr int PACKK_LDS = 2 * 9 * PACKSPAN;
 constexpr int SWEEPK_LDS = 2 * 9 * KSPAN;  // elements of k_sweepk's LDS
-constexpr int CELL_CHUNK = 1;  // cells each thread of the cell update walks along i
 
 template <typename R, bool B0V, bool ENT>
 __device__ __forceinline__ void k_sweepk_part(const SweepArgs &a, const int bx, const int by,
@@ -2093,7 +2092,6 @@ struct CellArgs {
   Geo geo;
   B0c b0;
   const double *b0a;       // per-point B0 (b0_mode 2), else null
-  int spherical;
   const double *X, *Xp;    // X^n, X^{n-1}
   double *Xn;              // X^{n+1} (aliases Xp: each cell reads before it writes)
   float *Xn32;             // FP32 copy of X^{n+1} (FP32-bulk form), else null
@@ -2132,7 +2130,16 @@ __device__ __forceinline__ void globalize(CellArgs &a) {
 // src/solver_func.c:2117-2135; spherical sources
 // src/spherical/spherical_general.c:605-688) plus the next step's CFL dt and
 // |div B| (src/solver_func.c:255-343).
-template <typename R, bool B0V>
+//
+// SPH: the grid has the spherical source terms.  A form of its own for each
+// kind: the terms cost a Cartesian grid 62 registers in FP64 (193 -> 131, a
+// third wave per SIMD) and 34 in FP32-bulk (162 -> 128, a fourth), and a
+// spherical grid, where they were read behind a branch on a.spherical, a second
+// wait for memory.  Bound by HBM: 256^3 1.46 -> 1.32 ms FP64 and 0.93 ->
+// 0.90 ms FP32-bulk (4.6 and 4.8 TB/s); shell 192x96x192 FP32-bulk 0.343 ->
+// 0.252 ms, sphere 128x128x256 FP64 0.445 -> 0.434 ms.  One wave more
+// asked for spills: 1.35, 1.74 ms at 256^3.
+template <typename R, bool B0V, bool SPH>
 __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, const int by,
                                        const int bz) {
   if (halted(a.sc)) return;
@@ -2141,15 +2148,10 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
   const Geo &G = a.geo;
   int k, j;
   const bool valid = row_point(g.s[2], g.e[2], g.s[1], g.e[1], bx, k, j);
-  // each thread walks CELL_CHUNK cells along i, so the i-face values a cell
-  // shares with the next (fluxes, face B) are re-read from cache, not HBM
-  const int i0 = g.s[0] + bz * CELL_CHUNK;
-  const int i1 = min(i0 + CELL_CHUNK, g.e[0] + 1);
+  const int i = g.s[0] + bz;
   double dtc = INFINITY, divb = 0.0;
   bool bad = false;
-  if (valid)
-#pragma unroll 1
-  for (int i = i0; i < i1; i++) {
+  if (valid) {
     const long c = i * g.st[0] + j * g.st[1] + k;
     const int idx[3] = {i, j, k};
     // the entropy channel's inputs, first, so that the loads of every other
@@ -2248,7 +2250,7 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
     for (int m = 0; m < 3; m++) bnew[m] = cell_b_of(bf[m][0], bf[m][1], G, idx[m], m);
 
     double SH[3] = {0.0, 0.0, 0.0}, SB[3] = {0.0, 0.0, 0.0};
-    if (a.spherical) {
+    if constexpr (SPH) {
       const double cc = a.sc->c;
       double xp[5];
 #pragma unroll
@@ -2373,17 +2375,17 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
   }
 }
 
-template <typename R, bool B0V>
+template <typename R, bool B0V, bool SPH>
 __global__ __launch_bounds__(256) void k_cell(CellArgs a, int gx, int gy, int gz) {
   int bx, by, bz;
   (void)gy;
   by = 0;
   if (!xcd_patch(gx, gz, bx, bz)) return;
-  k_cell_body<R, B0V>(a, bx, by, bz);
+  k_cell_body<R, B0V, SPH>(a, bx, by, bz);
 }
 
 // one launch for many grids: block w runs work-list entry w (argument set, block)
-template <typename R, bool B0V>
+template <typename R, bool B0V, bool SPH>
 __global__ __launch_bounds__(256) void k_cell_batch(const CellArgs *__restrict__ args,
                                                     const WorkItem *__restrict__ work, int nwork) {
   int w;
@@ -2393,7 +2395,7 @@ __global__ __launch_bounds__(256) void k_cell_batch(const CellArgs *__restrict__
   const int bx = __builtin_amdgcn_readfirstlane(work[w].bx);
   const int by = __builtin_amdgcn_readfirstlane(work[w].by);
   const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
-  k_cell_body<R, B0V>(batch_args(args, arg), bx, by, bz);
+  k_cell_body<R, B0V, SPH>(batch_args(args, arg), bx, by, bz);
 }
 
 // CFL dt and |div B| of the current state (prologue; src/solver_func.c:255-343)
@@ -4196,8 +4198,8 @@ void resolve_timers(gk_solver *s) {
 // id order (the k_pole_* and k_ring_* stages exist on pole ring-averaged grids)
 enum StageKernel {
   SK_BEGIN = 0, SK_SWEEP_I, SK_VSTRIP_I, SK_SWEEP_J, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_I, SK_EMF_J,
-  SK_EMF_K, SK_EMF_IS, SK_EMF_JS, SK_POLE_E, SK_CT, SK_POLE_B, SK_CELL, SK_RING_ROWS,
-  SK_RING_CURL, SK_RING_FIX, SK_RING_MAGS, SK_GHOST, SK_RING_DT, SK_COUNT,
+  SK_EMF_K, SK_EMF_IS, SK_EMF_JS, SK_POLE_E, SK_CT, SK_POLE_B, SK_CELL, SK_CELL_SPH,
+  SK_RING_ROWS, SK_RING_CURL, SK_RING_FIX, SK_RING_MAGS, SK_GHOST, SK_RING_DT, SK_COUNT,
   // stages of a small grid stepped alone (never in a batch): all sweeps and
   // all edge fields in one launch each, timed under the first stage's name
   SK_SWEEPS = SK_COUNT, SK_EDGES, SK_ALL
@@ -4205,7 +4207,7 @@ enum StageKernel {
 static const char *const sk_name[SK_ALL] = {
     "k_begin", "k_sweep_i", "k_vstrip_i", "k_sweep_j", "k_vstrip_j", "k_sweep_k", "k_sweep_k", "k_krem_k", "k_emf_i",
     "k_emf_j", "k_emf_k", "k_emf_i_tiles", "k_emf_j_tiles", "k_pole_e", "k_ct", "k_pole_b",
-    "k_cell", "k_ring_rows", "k_ring_curl", "k_ring_fix", "k_ring_mags", "k_ghost",
+    "k_cell", "k_cell", "k_ring_rows", "k_ring_curl", "k_ring_fix", "k_ring_mags", "k_ghost",
     "k_ring_dt", "k_sweep_i", "k_emf_i"};
 
 static_assert(sizeof(SweepsArgs) + 64 <= 4096 && sizeof(EdgesArgs) + 64 <= 4096, "kernel arguments");
@@ -4232,7 +4234,7 @@ static size_t stage_arg_size(int kid) {
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return sizeof(EmfArgs);
     case SK_CT: return sizeof(CtArgs);
-    case SK_CELL: return sizeof(CellArgs);
+    case SK_CELL: case SK_CELL_SPH: return sizeof(CellArgs);
     case SK_GHOST: return sizeof(GhostArgs);
     case SK_RING_DT: return sizeof(DtArgs);
     case SK_POLE_E: case SK_POLE_B: case SK_RING_ROWS: case SK_RING_CURL: case SK_RING_FIX:
@@ -4251,7 +4253,7 @@ static const void *stage_arg_ptr(int kid, const StageArgs &u) {
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return &u.em;
     case SK_CT: return &u.ct;
-    case SK_CELL: return &u.ce;
+    case SK_CELL: case SK_CELL_SPH: return &u.ce;
     case SK_GHOST: return &u.gh;
     case SK_RING_DT: return &u.dt;
     case SK_POLE_E: case SK_POLE_B: case SK_RING_ROWS: case SK_RING_CURL: case SK_RING_FIX:
@@ -4594,7 +4596,6 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
     a.b0 = s->b0;
     a.b0a = s->b0a;
   a.b0a = s->b0a;
-    a.spherical = s->spherical;
     a.X = X;
     a.Xp = Xp;
     a.Xn = Xn;
@@ -4623,8 +4624,8 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
         a.skip[3] = Ee[1];
       }
     }
-    L.kid = SK_CELL;
-    L.grid = dim3(row_blocks(S[2], Ee[2], S[1], Ee[1]), 1, (s->ni + CELL_CHUNK - 1) / CELL_CHUNK);
+    L.kid = s->spherical ? SK_CELL_SPH : SK_CELL;
+    L.grid = dim3(row_blocks(S[2], Ee[2], S[1], Ee[1]), 1, s->ni);
     L.u.ce = a;
     out.push_back(L);
   }
@@ -4702,7 +4703,7 @@ static void launch_one(const Launch &L, hipStream_t st) {
   const dim3 blk(64, 4);
   const int gx = L.grid.x, gy = L.grid.y, gz = L.grid.z;
   // decoded by xcd_patch (cell update, CT, cell B) or xcd_block (the others)
-  const bool patch = L.kid == SK_CT || L.kid == SK_CELL;
+  const bool patch = L.kid == SK_CT || L.kid == SK_CELL || L.kid == SK_CELL_SPH;
   const int total = patch ? patch_blocks(L.grid) : gx * gy * gz;
   const dim3 g1((total + NXCD - 1) / NXCD * NXCD);
   switch (L.kid) {
@@ -4720,7 +4721,8 @@ static void launch_one(const Launch &L, hipStream_t st) {
     case SK_EMF_IS: k_emf_stage<0, R, B0V, UT><<<g1, dim3(64), 0, st>>>(L.u.em, gx, gy, gz); break;
     case SK_EMF_JS: k_emf_stage<1, R, B0V, UT><<<g1, dim3(64), 0, st>>>(L.u.em, gx, gy, gz); break;
     case SK_CT: k_ct<R><<<g1, blk, 0, st>>>(L.u.ct, gx, gy, gz); break;
-    case SK_CELL: k_cell<R, B0V><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
+    case SK_CELL: k_cell<R, B0V, false><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
+    case SK_CELL_SPH: k_cell<R, B0V, true><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
     case SK_GHOST: k_ghost<<<g1, blk, 0, st>>>(L.u.gh, gx, gy, gz); break;
     case SK_POLE_E: k_pole_e<R><<<L.grid, dim3(64), 0, st>>>(L.u.rg); break;
     case SK_POLE_B: k_pole_b<<<L.grid, dim3(256), 0, st>>>(L.u.rg); break;
@@ -4753,7 +4755,8 @@ static void launch_batch(int kid, const void *args, const WorkItem *work, int nw
     case SK_EMF_IS: k_emf_stage_batch<0, R, B0V, UT><<<nblocks, dim3(64), 0, st>>>((const EmfArgs *)args, work, nwork); break;
     case SK_EMF_JS: k_emf_stage_batch<1, R, B0V, UT><<<nblocks, dim3(64), 0, st>>>((const EmfArgs *)args, work, nwork); break;
     case SK_CT: k_ct_batch<R><<<nblocks, blk, 0, st>>>((const CtArgs *)args, work, nwork); break;
-    case SK_CELL: k_cell_batch<R, B0V><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
+    case SK_CELL: k_cell_batch<R, B0V, false><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
+    case SK_CELL_SPH: k_cell_batch<R, B0V, true><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
     case SK_GHOST: k_ghost_batch<<<nblocks, blk, 0, st>>>((const GhostArgs *)args, work, nwork); break;
     case SK_POLE_E: k_pole_e_batch<R><<<nblocks, dim3(64), 0, st>>>((const RingArgs *)args, work, nwork); break;
     case SK_POLE_B: k_pole_b_batch<<<nblocks, dim3(256), 0, st>>>((const RingArgs *)args, work, nwork); break;
@@ -5293,7 +5296,7 @@ static void solo_order(int kid, dim3 gr, int idx, std::vector<WorkItem> &out) {
     case SK_EMF_JS: case SK_GHOST:
       mode = 1;
       break;
-    case SK_CT: case SK_CELL:
+    case SK_CT: case SK_CELL: case SK_CELL_SPH:
       mode = gy == 1 ? 2 : 0;
       break;
     default:  // SK_VSTRIP_I, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_K, the ring stages
