@@ -186,6 +186,25 @@ __device__ __forceinline__ bool halted(const Scal *sc) { return sc && sc->halt; 
 // 0.553, 1.01, 0.131 -> 0.390 / 0.392 / 0.533, 0.93, 0.121 ms.
 __device__ __forceinline__ bool carries_entropy(const Scal *sc) { return sc->ent != 0; }
 
+// element `o` of what starts at p, which is the same in all lanes: the byte
+// offset stays a 32-bit lane value beside a scalar base (one register instead
+// of two per address, no 64-bit add).  For offsets within a row or a plane: a
+// plane past 4 GiB would be a grid of terabytes.
+template <typename T>
+__device__ __forceinline__ T *lane(T *p, unsigned o) {
+  return (T *)((char *)p + o * (unsigned)sizeof(T));
+}
+template <typename T>
+__device__ __forceinline__ const T *lane(const T *p, unsigned o) {
+  return (const T *)((const char *)p + o * (unsigned)sizeof(T));
+}
+
+// the same offset as a value of its own: the compiler folds a 32-bit offset
+// into an access only where it is made in the block of the access
+__device__ __forceinline__ unsigned here(unsigned o) {
+  asm("" : "+v"(o));
+  return o;
+}
 __device__ __forceinline__ double geo3(const Geo &g, int q, int i, int j, int k) {
   return g.g[q][0][i] * g.g[q][1][j] * g.g[q][2][k];
 }
@@ -2063,6 +2082,95 @@ __device__ __forceinline__ void k_ct_body(const CtArgs &a, const int bx, const i
   }
 }
 
+// The same update by threads that walk CT_CHUNK points along i (FP64 grids from
+// CT_WALK cells): E_j and E_k at i + 1 are the next point's, and the row and
+// column factors are read once, 12 loads a point instead of 27.  The plain form
+// is bound by its load instructions (address unit 83 % busy at 3.7 of 6.2
+// TB/s): 256^3 0.369 -> 0.329 ms, sphere 128x128x256 0.098 -> 0.088, 128^3 0.052
+// -> 0.050.  Below that the launch
+// is too short to fill the chip with a quarter of the threads (96x72x60 0.0175 ->
+// 0.0192 ms, 32^3 0.007 -> 0.011), and in FP32-bulk, where the stores weigh more,
+// it gives 2 % at 256^3 and takes as much from an ensemble of small grids.
+constexpr int CT_CHUNK = 4;
+constexpr double CT_WALK = 1e6;
+
+__device__ __forceinline__ void k_ct_walk_body(const CtArgs &a, const int bx, const int by,
+                                               const int bz) {
+  if (halted(a.sc)) return;
+  const Grid &g = a.g;
+  (void)by;
+  int k, j;
+  if (!row_point(g.s[2], g.e[2] + 1, g.s[1], g.e[1] + 1, bx, k, j)) return;
+  const int i0 = g.s[0] + bz * CT_CHUNK, i1 = min(i0 + CT_CHUNK, g.e[0] + 2);
+  long ip = i0 * g.st[0];
+  unsigned c = j * (unsigned)g.st[1] + k;  // the point in its plane
+  const long SI = g.st[0], SJ = g.st[1];
+  const double dt = a.sc->dt;
+  const double *Ei = (const double *)a.E, *Ej = Ei + g.fs, *Ek = Ei + 2 * g.fs;
+  const Geo &G = a.geo;
+  const bool aj = j <= g.e[1], ak = k <= g.e[2];
+  // the row and column factors of the edges and faces around the point: the
+  // same at every i
+  const double *const *gi = G.g[GK_G_EDGE_I], *const *gj = G.g[GK_G_EDGE_J],
+               *const *gk = G.g[GK_G_EDGE_K], *const *fi = G.g[GK_G_FACE_I],
+               *const *fj = G.g[GK_G_FACE_J], *const *fk = G.g[GK_G_FACE_K];
+  const double gi1 = *lane(gi[1], j), gi1_j = *lane(gi[1] + 1, j), gi2 = *lane(gi[2], k),
+               gi2_k = *lane(gi[2] + 1, k);
+  const double gj1 = *lane(gj[1], j), gj2 = *lane(gj[2], k), gj2_k = *lane(gj[2] + 1, k);
+  const double gk1 = *lane(gk[1], j), gk1_j = *lane(gk[1] + 1, j), gk2 = *lane(gk[2], k);
+  const double fi1 = *lane(fi[1], j), fi2 = *lane(fi[2], k), fj1 = *lane(fj[1], j),
+               fj2 = *lane(fj[2], k), fk1 = *lane(fk[1], j), fk2 = *lane(fk[2], k);
+  // E_j, E_k and their edges at i: what the last point read at i + 1
+  double ej = *lane(Ej + ip, c), ej_k = *lane(Ej + ip + 1, c), ek = *lane(Ek + ip, c),
+         ek_j = *lane(Ek + ip + SJ, c);
+#pragma unroll 1
+  for (int i = i0; i < i1; i++, ip += SI) {
+    c = here(c);
+    const bool ai = i <= g.e[0];
+    // every input of the point is read before the first store, so the wave
+    // waits for memory once; neighbour indices stay inside the box for
+    // i, j, k <= e + 1
+    const double ei = *lane(Ei + ip, c), ei_j = *lane(Ei + ip + SJ, c),
+                 ei_k = *lane(Ei + ip + 1, c);
+    const double ej_i = *lane(Ej + ip + SI, c), ej_ik = *lane(Ej + ip + SI + 1, c),
+                 ek_i = *lane(Ek + ip + SI, c), ek_ij = *lane(Ek + ip + SI + SJ, c);
+    const double bi = ld_nt(lane(a.B + ip, c)), bj = ld_nt(lane(a.B + g.fs + ip, c)),
+                 bk = ld_nt(lane(a.B + 2 * g.fs + ip, c));
+    const double li = gi[0][i] * gi1 * gi2, li_j = gi[0][i] * gi1_j * gi2,
+                 li_k = gi[0][i] * gi1 * gi2_k;
+    const double lj = gj[0][i] * gj1 * gj2, lj_i = gj[0][i + 1] * gj1 * gj2,
+                 lj_k = gj[0][i] * gj1 * gj2_k;
+    const double lk = gk[0][i] * gk1 * gk2, lk_i = gk[0][i + 1] * gk1 * gk2,
+                 lk_j = gk[0][i] * gk1_j * gk2;
+    const double si = fi[0][i] * fi1 * fi2, sj = fj[0][i] * fj1 * fj2, sk = fk[0][i] * fk1 * fk2;
+    if (aj && ak) {  // B_i on faces i = is..ie+1
+      c = here(c);
+      const double d = (ek_j * lk_j - ek * lk) -
+                       (ej_k * lj_k - ej * lj);
+      const double b = bi - dt * d / si;
+      st_nt(lane(a.Bn + ip, c), b);
+    }
+    if (ai && ak) {  // B_j on faces j = js..je+1
+      c = here(c);
+      const double d = (ei_k * li_k - ei * li) -
+                       (ek_i * lk_i - ek * lk);
+      const double b = bj - dt * d / sj;
+      st_nt(lane(a.Bn + g.fs + ip, c), b);
+    }
+    if (ai && aj) {  // B_k on faces k = ks..ke+1
+      c = here(c);
+      const double d = (ej_i * lj_i - ej * lj) -
+                       (ei_j * li_j - ei * li);
+      const double b = bk - dt * d / sk;
+      st_nt(lane(a.Bn + 2 * g.fs + ip, c), b);
+    }
+    ej = ej_i;
+    ej_k = ej_ik;
+    ek = ek_i;
+    ek_j = ek_ij;
+  }
+}
+
 template <typename R>
 __global__ __launch_bounds__(256) void k_ct(CtArgs a, int gx, int gy, int gz) {
   int bx, by, bz;
@@ -2084,6 +2192,27 @@ __global__ __launch_bounds__(256) void k_ct_batch(const CtArgs *__restrict__ arg
   const int by = __builtin_amdgcn_readfirstlane(work[w].by);
   const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
   k_ct_body<R>(batch_args(args, arg), bx, by, bz);
+}
+
+__global__ __launch_bounds__(256) void k_ct_walk(CtArgs a, int gx, int gy, int gz) {
+  int bx, by, bz;
+  (void)gy;
+  by = 0;
+  if (!xcd_patch(gx, gz, bx, bz)) return;
+  k_ct_walk_body(a, bx, by, bz);
+}
+
+// one launch for many grids: block w runs work-list entry w (argument set, block)
+__global__ __launch_bounds__(256) void k_ct_walk_batch(const CtArgs *__restrict__ args,
+                                                    const WorkItem *__restrict__ work, int nwork) {
+  int w;
+  if (!xcd_item(nwork, w)) return;
+  // uniform per block: keep the argument set in scalar registers
+  const int arg = __builtin_amdgcn_readfirstlane(work[w].arg);
+  const int bx = __builtin_amdgcn_readfirstlane(work[w].bx);
+  const int by = __builtin_amdgcn_readfirstlane(work[w].by);
+  const int bz = __builtin_amdgcn_readfirstlane(work[w].bz);
+  k_ct_walk_body(batch_args(args, arg), bx, by, bz);
 }
 
 // ---------------------------------------------------------------------------
@@ -4198,7 +4327,7 @@ void resolve_timers(gk_solver *s) {
 // id order (the k_pole_* and k_ring_* stages exist on pole ring-averaged grids)
 enum StageKernel {
   SK_BEGIN = 0, SK_SWEEP_I, SK_VSTRIP_I, SK_SWEEP_J, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_I, SK_EMF_J,
-  SK_EMF_K, SK_EMF_IS, SK_EMF_JS, SK_POLE_E, SK_CT, SK_POLE_B, SK_CELL, SK_CELL_SPH,
+  SK_EMF_K, SK_EMF_IS, SK_EMF_JS, SK_POLE_E, SK_CT, SK_CT_WALK, SK_POLE_B, SK_CELL, SK_CELL_SPH,
   SK_RING_ROWS, SK_RING_CURL, SK_RING_FIX, SK_RING_MAGS, SK_GHOST, SK_RING_DT, SK_COUNT,
   // stages of a small grid stepped alone (never in a batch): all sweeps and
   // all edge fields in one launch each, timed under the first stage's name
@@ -4206,7 +4335,7 @@ enum StageKernel {
 };
 static const char *const sk_name[SK_ALL] = {
     "k_begin", "k_sweep_i", "k_vstrip_i", "k_sweep_j", "k_vstrip_j", "k_sweep_k", "k_sweep_k", "k_krem_k", "k_emf_i",
-    "k_emf_j", "k_emf_k", "k_emf_i_tiles", "k_emf_j_tiles", "k_pole_e", "k_ct", "k_pole_b",
+    "k_emf_j", "k_emf_k", "k_emf_i_tiles", "k_emf_j_tiles", "k_pole_e", "k_ct", "k_ct", "k_pole_b",
     "k_cell", "k_cell", "k_ring_rows", "k_ring_curl", "k_ring_fix", "k_ring_mags", "k_ghost",
     "k_ring_dt", "k_sweep_i", "k_emf_i"};
 
@@ -4233,7 +4362,7 @@ static size_t stage_arg_size(int kid) {
       return sizeof(SweepArgs);
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return sizeof(EmfArgs);
-    case SK_CT: return sizeof(CtArgs);
+    case SK_CT: case SK_CT_WALK: return sizeof(CtArgs);
     case SK_CELL: case SK_CELL_SPH: return sizeof(CellArgs);
     case SK_GHOST: return sizeof(GhostArgs);
     case SK_RING_DT: return sizeof(DtArgs);
@@ -4252,7 +4381,7 @@ static const void *stage_arg_ptr(int kid, const StageArgs &u) {
       return &u.sw;
     case SK_EMF_I: case SK_EMF_J: case SK_EMF_K: case SK_EMF_IS: case SK_EMF_JS:
       return &u.em;
-    case SK_CT: return &u.ct;
+    case SK_CT: case SK_CT_WALK: return &u.ct;
     case SK_CELL: case SK_CELL_SPH: return &u.ce;
     case SK_GHOST: return &u.gh;
     case SK_RING_DT: return &u.dt;
@@ -4577,8 +4706,10 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
     a.Bn32 = f32 ? s->B32[r.b_n] : nullptr;
     a.E = s->E;
     a.sc = s->sc;
-    L.kid = SK_CT;
-    L.grid = dim3(row_blocks(S[2], Ee[2] + 1, S[1], Ee[1] + 1), 1, s->ni + 1);
+    const bool walk = !f32 && (double)s->ni * s->nj * s->nk >= CT_WALK;
+    L.kid = walk ? SK_CT_WALK : SK_CT;
+    L.grid = dim3(row_blocks(S[2], Ee[2] + 1, S[1], Ee[1] + 1), 1,
+                  walk ? s->ni / CT_CHUNK + 1 : s->ni + 1);
     L.u.ct = a;
     out.push_back(L);
   }
@@ -4703,7 +4834,7 @@ static void launch_one(const Launch &L, hipStream_t st) {
   const dim3 blk(64, 4);
   const int gx = L.grid.x, gy = L.grid.y, gz = L.grid.z;
   // decoded by xcd_patch (cell update, CT, cell B) or xcd_block (the others)
-  const bool patch = L.kid == SK_CT || L.kid == SK_CELL || L.kid == SK_CELL_SPH;
+  const bool patch = L.kid == SK_CT || L.kid == SK_CT_WALK || L.kid == SK_CELL || L.kid == SK_CELL_SPH;
   const int total = patch ? patch_blocks(L.grid) : gx * gy * gz;
   const dim3 g1((total + NXCD - 1) / NXCD * NXCD);
   switch (L.kid) {
@@ -4721,6 +4852,7 @@ static void launch_one(const Launch &L, hipStream_t st) {
     case SK_EMF_IS: k_emf_stage<0, R, B0V, UT><<<g1, dim3(64), 0, st>>>(L.u.em, gx, gy, gz); break;
     case SK_EMF_JS: k_emf_stage<1, R, B0V, UT><<<g1, dim3(64), 0, st>>>(L.u.em, gx, gy, gz); break;
     case SK_CT: k_ct<R><<<g1, blk, 0, st>>>(L.u.ct, gx, gy, gz); break;
+    case SK_CT_WALK: k_ct_walk<<<g1, blk, 0, st>>>(L.u.ct, gx, gy, gz); break;
     case SK_CELL: k_cell<R, B0V, false><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
     case SK_CELL_SPH: k_cell<R, B0V, true><<<g1, blk, 0, st>>>(L.u.ce, gx, gy, gz); break;
     case SK_GHOST: k_ghost<<<g1, blk, 0, st>>>(L.u.gh, gx, gy, gz); break;
@@ -4755,6 +4887,7 @@ static void launch_batch(int kid, const void *args, const WorkItem *work, int nw
     case SK_EMF_IS: k_emf_stage_batch<0, R, B0V, UT><<<nblocks, dim3(64), 0, st>>>((const EmfArgs *)args, work, nwork); break;
     case SK_EMF_JS: k_emf_stage_batch<1, R, B0V, UT><<<nblocks, dim3(64), 0, st>>>((const EmfArgs *)args, work, nwork); break;
     case SK_CT: k_ct_batch<R><<<nblocks, blk, 0, st>>>((const CtArgs *)args, work, nwork); break;
+    case SK_CT_WALK: k_ct_walk_batch<<<nblocks, blk, 0, st>>>((const CtArgs *)args, work, nwork); break;
     case SK_CELL: k_cell_batch<R, B0V, false><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
     case SK_CELL_SPH: k_cell_batch<R, B0V, true><<<nblocks, blk, 0, st>>>((const CellArgs *)args, work, nwork); break;
     case SK_GHOST: k_ghost_batch<<<nblocks, blk, 0, st>>>((const GhostArgs *)args, work, nwork); break;
@@ -5296,7 +5429,7 @@ static void solo_order(int kid, dim3 gr, int idx, std::vector<WorkItem> &out) {
     case SK_EMF_JS: case SK_GHOST:
       mode = 1;
       break;
-    case SK_CT: case SK_CELL: case SK_CELL_SPH:
+    case SK_CT: case SK_CT_WALK: case SK_CELL: case SK_CELL_SPH:
       mode = gy == 1 ? 2 : 0;
       break;
     default:  // SK_VSTRIP_I, SK_VSTRIP_J, SK_SWEEP_K, SK_PACK_K, SK_KREM, SK_EMF_K, the ring stages
