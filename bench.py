@@ -40,12 +40,13 @@ def log(msg):
 def kernel_alg_bytes(name, n):
     """Compulsory HBM bytes of one launch of a stage kernel on an n^3 grid
     (each distinct input value read once, each output written once, 8 B per
-    value).  Counts follow the kernel's own inputs and outputs."""
+    value).  Counts follow the kernel's own inputs and outputs; the workload's
+    p_S is 0 everywhere, so the entropy channel moves nothing."""
     N = n + 9
     full_faces = (n + 1) * n * n
     if name.startswith("k_sweep_"):
-        # full faces: X^n, X^{n-1} (6+6), cell B at n, n-1 (3+3), face-normal
-        # B (1) in; 9 fluxes + 2 face velocities out.  The transverse
+        # full faces: X^n, X^{n-1} (5+5), cell B at n, n-1 (3+3), face-normal
+        # B (1) in; 8 fluxes + 2 face velocities out.  The transverse
         # extension (8 extra rows) only forms the 2 face velocities: 2+2 in,
         # 2 out.
         nf = n + 1
@@ -57,7 +58,7 @@ def kernel_alg_bytes(name, n):
                 nf -= rem
         full = nf * n * n
         ext_faces = nf * (N - 1 - n) * n
-        return 8 * (full * 30 + ext_faces * 6)
+        return 8 * (full * 27 + ext_faces * 6)
     if name.startswith("k_emf_"):
         # per edge: 2 face velocities, 2 face-B (n, n-1 each), density at n, n-1
         # in, 1 EMF out
@@ -66,14 +67,12 @@ def kernel_alg_bytes(name, n):
         # 3 face-B in, 3 EMF in, 3 face-B out
         return 8 * 9 * full_faces
     if name == "k_cell":
-        # 27 face fluxes, X^n (6), cell B^n (3), face B^{n+1} (3) in; X^{n+1} (6)
+        # 24 face fluxes, X^n (5), cell B^n (3), face B^{n+1} (3) in; X^{n+1} (5)
         # and cell B^{n+1} (3) out
-        return 8 * n ** 3 * 48
+        return 8 * n ** 3 * 43
     if name == "k_ghost":
-        return 8 * 2 * 9 * (N ** 3 - n ** 3)
-    if name == "k_mags":
-        # cell B of the points outside the active cells: 3 face fields in, 3 out
-        return 8 * 6 * ((N - 1) ** 3 - n ** 3)
+        # X and B copied, cell B of the points outside the active cells out
+        return 8 * (2 * 8 * (N ** 3 - n ** 3) + 3 * ((N - 1) ** 3 - n ** 3))
     return 0
 
 

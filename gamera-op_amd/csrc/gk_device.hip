@@ -2264,8 +2264,9 @@ __device__ __forceinline__ void globalize(CellArgs &a) {
 // kind: the terms cost a Cartesian grid 62 registers in FP64 (193 -> 131, a
 // third wave per SIMD) and 34 in FP32-bulk (162 -> 128, a fourth), and a
 // spherical grid, where they were read behind a branch on a.spherical, a second
-// wait for memory.  Bound by HBM: 256^3 1.46 -> 1.32 ms FP64 and 0.93 ->
-// 0.90 ms FP32-bulk (4.6 and 4.8 TB/s); shell 192x96x192 FP32-bulk 0.343 ->
+// wait for memory.  Bound by its load instructions (90 a cell in FP64, address
+// unit 85 % busy) at 4.6 and 4.8 of 6.2 TB/s: 256^3 1.46 -> 1.32 ms FP64 and
+// 0.93 -> 0.89 ms FP32-bulk; shell 192x96x192 FP32-bulk 0.343 ->
 // 0.252 ms, sphere 128x128x256 FP64 0.445 -> 0.434 ms.  One wave more
 // asked for spills: 1.35, 1.74 ms at 256^3.
 template <typename R, bool B0V, bool SPH>
