@@ -3476,6 +3476,7 @@ struct gk_solver {
   int merge_sweeps;    // alone: all sweeps in one launch (k_sweeps)
   int merge_edges;     // alone: all edge fields in one launch, one edge per thread (k_edges)
   int merge_chunk;     // faces per thread in the marches of a merged launch
+  int merge_asked;     // the merged launches were set by GK_TUNE_MERGE: a length asked for keeps them
   double rho_floor, p_floor;  // positivity floors
   double grav[3];      // uniform gravity
   struct gk_batch *batch;  // batch that owns the stepping, if any
@@ -3634,6 +3635,18 @@ static hipError_t upload(gk_solver *s, void *dst, const void *src, size_t bytes)
   return e;
 }
 
+// Small grids stepped alone take all sweeps in one launch (k_sweeps) up to
+// 6e5 cells in FP64 and 1e6 in FP32-bulk, and all edge fields in one
+// (k_edges) up to 3e5 (ms per step with the launches apart / merged: 32^3
+// FP64 0.105 / 0.060; 48^3 0.143 / 0.108; 128x128x8 0.180 / 0.140; 64^3 0.208
+// / 0.175; 96x72x60 0.329 / 0.300; 96^3 0.509 / 0.530; FP32-bulk 64^3 0.146 /
+// 0.116, 80^3 0.283 / 0.232, 96^3 0.309 / 0.297; edges alone 64^3 0.194 /
+// 0.175, 96x72x60 0.086 / 0.088 ms).
+static bool merges_sweeps(const gk_solver *s) {
+  return (double)s->ni * s->nj * s->nk < (s->precision == 1 ? 1e6 : 6e5);
+}
+static bool merges_edges(const gk_solver *s) { return (double)s->ni * s->nj * s->nk < 3e5; }
+
 // Default march lengths by grid size (faces per thread in the i and j
 // sweeps, edges per thread in the edge-field kernels): smaller grids need
 // shorter marches, so that their columns are split over enough threads to
@@ -3644,13 +3657,7 @@ static hipError_t upload(gk_solver *s, void *dst, const void *src, size_t bytes)
 // default for every size, (32, 16), had cost 32^3 3.8x and 128x128x8 2.3x.
 // gk_autotune times the candidates on the grid itself.
 //
-// Small grids stepped alone take all sweeps in one launch (k_sweeps) up to
-// 6e5 cells in FP64 and 1e6 in FP32-bulk, and all edge fields in one
-// (k_edges) up to 3e5 (ms per step with the launches apart / merged: 32^3
-// FP64 0.105 / 0.060; 48^3 0.143 / 0.108; 128x128x8 0.180 / 0.140; 64^3 0.208
-// / 0.175; 96x72x60 0.329 / 0.300; 96^3 0.509 / 0.530; FP32-bulk 64^3 0.146 /
-// 0.116, 80^3 0.283 / 0.232, 96^3 0.309 / 0.297; edges alone 64^3 0.194 /
-// 0.175, 96x72x60 0.086 / 0.088 ms).  Merged marches share the chip, so they
+// Merged marches share the chip, so they
 // may be longer than a march that has it alone: 2 faces per thread best at
 // 32^3, 4 at 61x43x37, 8 at 48^3, 12 at 128x128x8 and above.
 static void default_shapes(gk_solver *s) {
@@ -3675,8 +3682,9 @@ static void default_shapes(gk_solver *s) {
     s->chunk = 2;
     s->emf_chunk = 2;
   }
-  s->merge_sweeps = n < (s->precision == 1 ? 1e6 : 6e5);
-  s->merge_edges = n < 3e5;
+  s->merge_sweeps = merges_sweeps(s);
+  s->merge_edges = merges_edges(s);
+  s->merge_asked = 0;
   s->merge_chunk = n < 5e4 ? 2 : n < 1e5 ? 4 : n < 1.25e5 ? 8 : 12;
 }
 
@@ -5322,18 +5330,29 @@ extern "C" int gk_set_tuning(gk_solver *s, int param, int value) {
   if (param == GK_TUNE_EMF_STAGE) {
     if (value < 0 || value > 3) return GK_ERR_ARG;
     s->emf_stage = value;
-    s->merge_edges = 0;  // a length or form asked for is the one that runs
+    // a length or form asked for is the one that runs, unless the merged
+    // launches were asked for too (so that all parameters read from one solver
+    // can be set on another, in any order)
+    if (!s->merge_asked) s->merge_edges = 0;
+    return GK_OK;
+  }
+  if (param == GK_TUNE_MERGE) {
+    const int has = (merges_sweeps(s) ? 1 : 0) | (merges_edges(s) ? 2 : 0);
+    if (value < 0 || (value & ~has)) return GK_ERR_ARG;
+    s->merge_sweeps = value & 1;
+    s->merge_edges = value >> 1;
+    s->merge_asked = 1;
     return GK_OK;
   }
   if (value < 1 || value > 4096) return GK_ERR_ARG;
   if (param == GK_TUNE_CHUNK) {
     s->chunk = value;
-    s->merge_sweeps = 0;
+    if (!s->merge_asked) s->merge_sweeps = 0;
     return GK_OK;
   }
   if (param == GK_TUNE_EMF_CHUNK) {
     s->emf_chunk = value;
-    s->merge_edges = 0;
+    if (!s->merge_asked) s->merge_edges = 0;
     return GK_OK;
   }
   return GK_ERR_ARG;
@@ -5344,6 +5363,7 @@ extern "C" int gk_get_tuning(const gk_solver *s, int param) {
   if (param == GK_TUNE_CHUNK) return s->chunk;
   if (param == GK_TUNE_EMF_CHUNK) return s->emf_chunk;
   if (param == GK_TUNE_EMF_STAGE) return s->emf_stage;
+  if (param == GK_TUNE_MERGE) return (s->merge_sweeps ? 1 : 0) | (s->merge_edges ? 2 : 0);
   return GK_ERR_ARG;
 }
 

@@ -192,6 +192,7 @@ def copy_calibrate(nbytes, reps=20):
 TUNE_CHUNK = 0
 TUNE_EMF_CHUNK = 1
 TUNE_EMF_STAGE = 2
+TUNE_MERGE = 3
 
 
 class GkError(RuntimeError):

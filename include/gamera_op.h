@@ -221,12 +221,18 @@ size_t gk_device_bytes(const gk_solver *s);
    about that length (within 1.5x of it).  GK_TUNE_EMF_STAGE: bit D (D = 0
    for E_i, 1 for E_j) runs that edge field over whole 64-edge tiles along
    k with its k-direction reconstructions staged in LDS (0..3; default 3 in
-   FP64, 2 in FP32-bulk).  Until one of these is set, a small grid stepped
-   alone runs all its sweeps (up to 6e5 cells, FP32-bulk 1e6) and all its
-   edge fields (up to 3e5 cells) in one launch each, which gk_kernel_times
-   lists as k_sweep_i and k_emf_i.  GK_ERR_STATE while the solver is in a
-   batch (the batch's launch tables hold its shapes). */
-enum { GK_TUNE_CHUNK = 0, GK_TUNE_EMF_CHUNK = 1, GK_TUNE_EMF_STAGE = 2 };
+   FP64, 2 in FP32-bulk).  GK_TUNE_MERGE: a small grid stepped alone runs
+   all its sweeps (bit 0; below 6e5 cells, FP32-bulk 1e6) and all its edge
+   fields (bit 1; below 3e5 cells) in one launch each, which gk_kernel_times
+   lists as k_sweep_i and k_emf_i.  Its bits are on by default on those grids,
+   and a bit a larger grid does not have is refused (GK_ERR_ARG).  While it has
+   not been set, setting one of the other three takes the launches it shapes
+   apart, so that what was asked for is what runs; once it has been, it stays,
+   and the values of all four read from one solver put another of its shape
+   into the same form whatever order they are set in.  GK_ERR_STATE while the
+   solver is in a batch (the batch's launch tables hold its shapes; a batch
+   never merges a grid's launches). */
+enum { GK_TUNE_CHUNK = 0, GK_TUNE_EMF_CHUNK = 1, GK_TUNE_EMF_STAGE = 2, GK_TUNE_MERGE = 3 };
 int gk_set_tuning(gk_solver *s, int param, int value);
 int gk_get_tuning(const gk_solver *s, int param);
 

@@ -1,0 +1,79 @@
+"""Launch shapes: what can be read from one solver can be set on another.
+
+A small grid runs its sweeps and its edge fields merged.  Which form runs shows
+in the stages that are timed: k_sweep_j and k_emf_k exist only apart.
+"""
+import itertools
+
+import pytest
+
+import gamera_op as go
+
+PARAMS = [go.TUNE_CHUNK, go.TUNE_EMF_CHUNK, go.TUNE_EMF_STAGE, go.TUNE_MERGE]
+
+
+def stages(S):
+    S.enable_timing(True)
+    S.step(1)
+    S.enable_timing(False)
+    return {k for k, v in S.kernel_times().items() if v > 0.0}
+
+
+def merged(S):
+    """(sweeps, edge fields) in one launch each"""
+    names = stages(S)
+    return "k_sweep_j" not in names, "k_emf_k" not in names
+
+
+@pytest.fixture
+def make():
+    made = []
+
+    def solver(precision=0, n=(16, 12, 10), kind=go.SINUSOID_SPHERE):
+        P = go.Problem(kind, 71, *n)
+        S = go.Solver(P, precision)
+        P.close()
+        made.append(S)
+        return S
+
+    yield solver
+    for S in made:
+        S.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("merge", [3, 2, 1, 0])
+def test_values_read_and_set_again(make, merge):
+    A = make()
+    assert A.get_tuning(go.TUNE_MERGE) == 3 and merged(A) == (True, True)
+    A.set_tuning(go.TUNE_MERGE, merge)
+    want = merged(A)
+    assert want == (bool(merge & 1), bool(merge & 2))
+    values = [A.get_tuning(p) for p in PARAMS]
+    for order in itertools.permutations(PARAMS):
+        B = make()
+        for p in order:
+            B.set_tuning(p, values[p])
+        assert [B.get_tuning(p) for p in PARAMS] == values, order
+        assert merged(B) == want, order
+
+
+@pytest.mark.gpu
+def test_a_length_alone_takes_the_launches_apart(make):
+    S = make(1)
+    S.set_tuning(go.TUNE_CHUNK, 4)
+    assert S.get_tuning(go.TUNE_MERGE) == 2 and merged(S) == (False, True)
+    S.set_tuning(go.TUNE_EMF_CHUNK, 4)
+    assert S.get_tuning(go.TUNE_MERGE) == 0 and merged(S) == (False, False)
+
+
+@pytest.mark.gpu
+def test_bits_a_grid_does_not_have_are_refused(make):
+    S = make(0, (70, 68, 66))  # 314160 cells: its sweeps merge, its edge fields do not
+    assert S.get_tuning(go.TUNE_MERGE) == 1
+    for bad in (-1, 2, 3, 4):
+        with pytest.raises(go.GkError):
+            S.set_tuning(go.TUNE_MERGE, bad)
+    assert S.get_tuning(go.TUNE_MERGE) == 1
+    S.set_tuning(go.TUNE_MERGE, 0)
+    assert merged(S) == (False, False)
