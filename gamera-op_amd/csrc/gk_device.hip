@@ -5871,13 +5871,17 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
   if (!s || trial_steps < 0) return GK_ERR_ARG;
   if (s->ready != 3 || s->batch) return GK_ERR_STATE;
   const TuneKey key{s->ni, s->nj, s->nk, s->spherical, s->precision};
+  const TunePick before{s->chunk, s->emf_chunk, s->emf_stage, s->merge_sweeps, s->merge_edges};
+  auto take = [&](const TunePick &p) {
+    s->chunk = p.chunk;
+    s->emf_chunk = p.emf_chunk;
+    s->emf_stage = p.emf_stage;
+    s->merge_sweeps = p.merge_sweeps;
+    s->merge_edges = p.merge_edges;
+  };
   for (auto &e : g_tune_cache)
     if (e.first == key) {
-      s->chunk = e.second.chunk;
-      s->emf_chunk = e.second.emf_chunk;
-      s->emf_stage = e.second.emf_stage;
-      s->merge_sweeps = e.second.merge_sweeps;
-      s->merge_edges = e.second.merge_edges;
+      take(e.second);
       if (best) *best = e.second.chunk;
       return GK_OK;
     }
@@ -5959,10 +5963,12 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
   float best_ms = 1e30f;
   // merged launches, where the grid has them, against the best march apart (the
   // march lengths are also what the grid takes inside a batch, which does not
-  // merge)
-  int merge_s = s->merge_sweeps, merge_e = s->merge_edges;
+  // merge).  They are tried by the grid's size, not by what the calling solver
+  // runs: the pick is kept for every later solver of the shape.
   float ms_s = 1e30f, ms_e = 1e30f;
-  if (rc == GK_OK && merge_s) rc = trial(ms_s);
+  s->merge_edges = merges_edges(s);
+  s->merge_sweeps = merges_sweeps(s);
+  if (rc == GK_OK && s->merge_sweeps) rc = trial(ms_s);
   s->merge_sweeps = 0;
   for (int c : cand) {
     if (rc != GK_OK) break;
@@ -5976,9 +5982,8 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
     }
   }
   s->chunk = pick;
-  merge_s = ms_s < best_ms;
-  s->merge_sweeps = merge_s;
-  if (rc == GK_OK && merge_e) rc = trial(ms_e);
+  s->merge_sweeps = ms_s < best_ms;
+  if (rc == GK_OK && s->merge_edges) rc = trial(ms_e);
   s->merge_edges = 0;
   best_ms = 1e30f;
   for (int c : cand_e) {
@@ -6010,19 +6015,15 @@ extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
       }
     }
   }
-  merge_e = ms_e < best_ms;
   s->timing = keep_timing;
   if (e0) (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);
   (void)hipFreeAsync(save, s->stream);
   (void)hipStreamSynchronize(s->stream);
-  s->merge_sweeps = merge_s;
-  s->merge_edges = merge_e;
+  const TunePick won{pick, pick_e, pick_s, s->merge_sweeps, ms_e < best_ms};
+  take(rc == GK_OK ? won : before);  // an error leaves the shapes as they were
   if (rc != GK_OK) return rc;
-  s->chunk = pick;
-  s->emf_chunk = pick_e;
-  s->emf_stage = pick_s;
-  g_tune_cache.push_back({key, TunePick{pick, pick_e, pick_s, merge_s, merge_e}});
+  g_tune_cache.push_back({key, won});
   if (best) *best = pick;
   return GK_OK;
 }

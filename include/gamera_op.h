@@ -240,10 +240,12 @@ int gk_get_tuning(const gk_solver *s, int param);
    trial_steps steps for each candidate march length of the sweeps and of the
    edge-field kernels and, on grids with whole 64-edge tiles along k, each
    GK_TUNE_EMF_STAGE setting, against the merged launches where the grid has
-   them; keeps the fastest of each (the sweeps' march
-   length is written to *best) and restores the state it started from, so
-   results do not depend on tuning.  Picks are cached per grid shape and
-   precision for the life of the process.  trial_steps = 0 only applies a
+   them (whatever GK_TUNE_MERGE says); keeps the fastest of each and restores
+   the state it started from, so results do not depend on tuning.  *best
+   receives the sweeps' march length apart, which is also what the grid takes
+   in a batch; GK_TUNE_MERGE tells whether they run merged.  Picks are cached
+   per grid shape and precision for the life of the process; after an error the
+   solver keeps the shapes it had.  trial_steps = 0 only applies a
    cached pick (*best = 0 when there is none) and times nothing. */
 int gk_autotune(gk_solver *s, int trial_steps, int *best);
 

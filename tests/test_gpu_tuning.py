@@ -77,3 +77,24 @@ def test_bits_a_grid_does_not_have_are_refused(make):
     assert S.get_tuning(go.TUNE_MERGE) == 1
     S.set_tuning(go.TUNE_MERGE, 0)
     assert merged(S) == (False, False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+def test_pick_does_not_depend_on_who_asked_first(make, precision):
+    """A solver taken apart by hand and then autotuned leaves the same pick for
+    later ones as one that was not touched: on these two grids of about 6000
+    cells (shapes no other test tunes) the merged launches are far ahead."""
+    n = (20, 18, 16 + precision)
+    A = make(precision, n)
+    for p in (go.TUNE_CHUNK, go.TUNE_EMF_CHUNK):
+        A.set_tuning(p, 4)
+    A.autotune(2)
+    B = make(precision, n)
+    assert B.autotune(0) > 0
+    for S in (A, B):
+        assert S.get_tuning(go.TUNE_MERGE) == 3 and merged(S) == (True, True)
+    assert [A.get_tuning(p) for p in PARAMS] == [B.get_tuning(p) for p in PARAMS]
+    C = make(precision, n)
+    C.set_tuning(go.TUNE_MERGE, 0)
+    assert C.autotune(0) > 0 and merged(C) == (True, True)
