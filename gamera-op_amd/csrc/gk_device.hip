@@ -5855,11 +5855,14 @@ extern "C" int gk_batch_step(gk_batch *b, int n) {
 // length on this grid and keeps the fastest.  The state (both time levels,
 // face and cell B, scalars, history rotation) is saved first and restored
 // afterwards, so results do not depend on tuning.  Picks are cached per
-// (ni, nj, nk, coord, precision) for the life of the process.
+// shape, coordinates and kernels (launch_group: precision, background field per
+// point, uniform tables; and the pole rings' extra stages) for the life of the
+// process.
 struct TuneKey {
-  int ni, nj, nk, coord, prec;
+  int ni, nj, nk, coord, group, ring;
   bool operator==(const TuneKey &o) const {
-    return ni == o.ni && nj == o.nj && nk == o.nk && coord == o.coord && prec == o.prec;
+    return ni == o.ni && nj == o.nj && nk == o.nk && coord == o.coord && group == o.group &&
+           ring == o.ring;
   }
 };
 struct TunePick {
@@ -5870,7 +5873,7 @@ static std::vector<std::pair<TuneKey, TunePick>> g_tune_cache;
 extern "C" int gk_autotune(gk_solver *s, int trial_steps, int *best) {
   if (!s || trial_steps < 0) return GK_ERR_ARG;
   if (s->ready != 3 || s->batch) return GK_ERR_STATE;
-  const TuneKey key{s->ni, s->nj, s->nk, s->spherical, s->precision};
+  const TuneKey key{s->ni, s->nj, s->nk, s->spherical, launch_group(s), s->ring};
   const TunePick before{s->chunk, s->emf_chunk, s->emf_stage, s->merge_sweeps, s->merge_edges};
   auto take = [&](const TunePick &p) {
     s->chunk = p.chunk;

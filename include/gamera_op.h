@@ -244,7 +244,8 @@ int gk_get_tuning(const gk_solver *s, int param);
    the state it started from, so results do not depend on tuning.  *best
    receives the sweeps' march length apart, which is also what the grid takes
    in a batch; GK_TUNE_MERGE tells whether they run merged.  Picks are cached
-   per grid shape and precision for the life of the process; after an error the
+   for the life of the process per grid shape, coordinates and kernels (precision, a
+   background field per point, one or several table classes, pole rings); after an error the
    solver keeps the shapes it had.  trial_steps = 0 only applies a
    cached pick (*best = 0 when there is none) and times nothing. */
 int gk_autotune(gk_solver *s, int trial_steps, int *best);

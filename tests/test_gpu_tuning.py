@@ -98,3 +98,16 @@ def test_pick_does_not_depend_on_who_asked_first(make, precision):
     C = make(precision, n)
     C.set_tuning(go.TUNE_MERGE, 0)
     assert C.autotune(0) > 0 and merged(C) == (True, True)
+
+
+@pytest.mark.gpu
+def test_pick_is_for_the_kernels_it_was_timed_on(make):
+    """A background field per point runs other kernels on the same shape."""
+    n = (22, 18, 14)
+    A = make(0, n)
+    assert A.autotune(1) > 0
+    B = make(0, n, go.VARYING_B0_BOX)
+    before = [B.get_tuning(p) for p in PARAMS]
+    assert B.autotune(0) == 0 and [B.get_tuning(p) for p in PARAMS] == before
+    C = make(0, n)
+    assert C.autotune(0) == A.get_tuning(go.TUNE_CHUNK)
