@@ -193,7 +193,11 @@ int gk_set_time(gk_solver *s, double time_sim);
    on for the launches of one stage only (name as gk_kernel_times reports it,
    e.g. "k_cell"; NULL: every stage), so that a timed run carries two events
    per step instead of two per launch; gk_enable_timing(s, 1) times every
-   stage again.  (No counterpart in the reference.) */
+   stage again.  A stage that runs inside another's launch (GK_TUNE_MERGE: the
+   sweeps of a small grid in k_sweep_i's, its edge fields in k_emf_i's; on
+   every grid k_mags, the cell B of the ghost cells, in k_ghost's) is listed
+   with that one; asked for by its own name, the whole launch is timed and
+   listed under the name asked for.  (No counterpart in the reference.) */
 int gk_enable_timing(gk_solver *s, int on);
 int gk_time_stage(gk_solver *s, const char *name);
 int gk_kernel_times(gk_solver *s, const char **names, double *ms, int *n);

@@ -111,3 +111,19 @@ def test_pick_is_for_the_kernels_it_was_timed_on(make):
     assert B.autotune(0) == 0 and [B.get_tuning(p) for p in PARAMS] == before
     C = make(0, n)
     assert C.autotune(0) == A.get_tuning(go.TUNE_CHUNK)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("merge", [3, 0])
+def test_every_stage_can_be_timed_by_name(make, merge):
+    """Stages that run inside another's launch answer to their own names too."""
+    S = make(0, (12, 10, 16))
+    S.set_tuning(go.TUNE_MERGE, merge)
+    for name in ("k_begin", "k_sweep_i", "k_sweep_j", "k_vstrip_j", "k_sweep_k", "k_emf_i", "k_emf_j",
+                 "k_emf_k", "k_ct", "k_cell", "k_ghost", "k_mags"):
+        S.time_stage(name)
+        S.step(2)
+        assert {k for k, v in S.kernel_times().items() if v > 0.0} == {name}, name
+    S.time_stage("no such stage")
+    S.step(1)
+    assert not any(S.kernel_times().values())
