@@ -37,12 +37,18 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def kernel_alg_bytes(name, n):
+def kernel_alg_bytes(name, n, merged=0):
     """Compulsory HBM bytes of one launch of a stage kernel on an n^3 grid
     (each distinct input value read once, each output written once, 8 B per
     value).  Counts follow the kernel's own inputs and outputs; the workload's
-    p_S is 0 everywhere, so the entropy channel moves nothing."""
+    p_S is 0 everywhere, so the entropy channel moves nothing.  merged: the
+    solver's TUNE_MERGE (small grids): k_sweep_i then is all three sweeps in one
+    launch, k_emf_i all three edge fields."""
     N = n + 9
+    if name == "k_sweep_i" and merged & 1:
+        return 3 * kernel_alg_bytes(name, n)
+    if name == "k_emf_i" and merged & 2:
+        return 3 * kernel_alg_bytes(name, n)
     full_faces = (n + 1) * n * n
     if name.startswith("k_sweep_"):
         # full faces: X^n, X^{n-1} (5+5), cell B at n, n-1 (3+3), face-normal
@@ -82,8 +88,8 @@ BREAKDOWN_STEPS = 10
 def run_form(args, precision):
     """Time one form of the step on the default workload; returns wall time,
     per-kernel HIP-event averages, device scalars, the final active state,
-    set-up/read-back times, the dominant stage and its HIP-event average over
-    the timed steps.  The per-stage breakdown comes from its own
+    set-up/read-back times, the dominant stage, its HIP-event average over
+    the timed steps and its compulsory bytes.  The per-stage breakdown comes from its own
     BREAKDOWN_STEPS steps before the timed ones, with events around every
     launch (about 0.12 ms per FP64 step at 256^3); the timed steps carry
     events around the dominant stage's launches only."""
@@ -128,8 +134,9 @@ def run_form(args, precision):
              "rhov1": (P.gas(0)[a, b, c] * P.gas(1)[a, b, c]),
              "Bi": P.gem(0)[4:5 + n, b, c].copy(), "Bj": P.gem(1)[a, 4:5 + n, c].copy(),
              "Bk": P.gem(2)[a, b, 4:5 + n].copy()}
+    alg = kernel_alg_bytes(dom, n, P.get_tuning(go.TUNE_MERGE))
     P.close()
-    return el, kt, sc, state, (t_open, t_fetch), dom, dom_ms
+    return el, kt, sc, state, (t_open, t_fetch), dom, dom_ms, alg
 
 
 def rel_l1(x, y):
@@ -141,10 +148,10 @@ def run_gpu(args):
     sys.path.insert(0, PKG)
     import gamera_op as go
 
-    el, kt, sc, st64, io, dom, dom_ms = run_form(args, 0)
+    el, kt, sc, st64, io, dom, dom_ms, alg = run_form(args, 0)
     fp32 = None
     if not args.no_fp32:
-        el32, kt32, sc32, st32, _, _, _ = run_form(args, 1)
+        el32, kt32, sc32, st32, _, _, _, _ = run_form(args, 1)
         cells = args.n ** 3
         fp32 = {"value": cells * args.steps / el32, "unit": "cell-updates/s",
                 "ms_per_step": el32 * 1e3 / args.steps, "speedup_vs_fp64": el / el32,
@@ -156,7 +163,7 @@ def run_gpu(args):
     log("bench: copy calibration")
     cbytes = 2 * 8 * (args.n + 9) ** 3 * 6  # read + write of six fields
     cms = go.copy_calibrate(cbytes // 2, 20)
-    return el, kt, sc, cbytes / (cms * 1e-3) / 1e9, fp32, io, dom, dom_ms
+    return el, kt, sc, cbytes / (cms * 1e-3) / 1e9, fp32, io, dom, dom_ms, alg
 
 
 RING_KERNELS = ("k_pole_e", "k_pole_b", "k_ring_rows", "k_ring_curl", "k_ring_fix",
@@ -593,12 +600,11 @@ def main():
         import serve
         preparer = serve.Preparer(args.serve_workers or None)
 
-    el, kt, sc, copy_gbs, fp32, io, dom, dom_ms = run_gpu(args)
+    el, kt, sc, copy_gbs, fp32, io, dom, dom_ms, alg = run_gpu(args)
     n = args.n
     cells = n ** 3
     value = cells * args.steps / el
     ms_step = el * 1e3 / args.steps
-    alg = kernel_alg_bytes(dom, n)
     achieved = alg / (dom_ms * 1e-3) / 1e9
     traffic = None
     tfile = os.path.join(ROOT, "profiles", f"{dom}_{n}cube_traffic.json")
