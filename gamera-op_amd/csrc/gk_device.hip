@@ -3658,6 +3658,36 @@ static bool merges_sweeps(const gk_solver *s) {
 }
 static bool merges_edges(const gk_solver *s) { return (double)s->ni * s->nj * s->nk < 3e5; }
 
+// rows of wk faces along k that a tile of the k sweep holds (1: not packed)
+static int pack_rows(int wk) { return wk <= 32 ? std::min(64 / wk, PACKSPAN / (wk + 7)) : 1; }
+
+// Faces per thread of the marches in a merged launch.  y: the faces its waves
+// take, per wave slot of the chip, each march wave's as many as it walks and one
+// for each k tile and strip wave.  The launch lasts a little over y faces' time,
+// and a march its faces and about one more (the cells it reads ahead of the first).
+// Marches that end with the launch, while the short waves fill the slots around
+// them, are best: longer ones outlast it, shorter ones read ahead more often.
+// 1.45 y - 1.2 is from a sweep of lengths 2 to 14 over 21 grids, 20^3 to 250x40x24, in
+// both forms: 0.6 % above the best length on average, 3.2 % at most.  ms per
+// step with lengths 2 / 4 / 6 / 8 / 10 / 12: FP64 32^3 (y 2.5) 0.0602 / 0.0603 /
+// 0.0641 / 0.0719 / 0.0778 / 0.0773, 48^3 (6.6) 0.1154 / 0.1091 / 0.1087 / 0.1069 /
+// 0.1064 / 0.1153, 128x128x8 (8.6) 0.1514 / 0.1501 / 0.1443 / 0.1391 / 0.1390 /
+// 0.1379; FP32-bulk 48^3 (3.3) 0.0747 / 0.0743 / 0.0790 / 0.0835 / 0.0849 / 0.0937,
+// 64x64x40 (5.2) 0.0970 / 0.0943 / 0.0937 / 0.0966 / 0.0993 / 0.1061.  Above 12, which
+// larger grids reach, a length gains 2 % at most and loses up to 5 %.
+static int merge_length(const gk_solver *s) {
+  const double ni = s->ni, nj = s->nj, nk = s->nk;
+  const int wk = s->nk + 1, rem = wk % 64;
+  const double rows = (ni + 2 * NGH) * nj;
+  double tiles = rows / pack_rows(wk);
+  if (wk > 32) tiles = rows * (wk / 64 + (wk >= 64 && rem < 32 ? rem / 64.0 : rem > 0));
+  const double marches = (nj + 2 * NGH) * nk / 64 * (ni + 1) + ni * nk / 64 * (nj + 1);
+  const double strips = 2 * NGH * ni / 64 * (nj + 1);
+  const double slots = 1024.0 * (s->precision == 1 ? MarchWaves<float>::n : MarchWaves<double>::n);
+  const double y = (marches + tiles + strips) / slots;
+  return std::max(2, std::min(12, (int)(1.45 * y - 0.7)));
+}
+
 // Default march lengths by grid size (faces per thread in the i and j
 // sweeps, edges per thread in the edge-field kernels): smaller grids need
 // shorter marches, so that their columns are split over enough threads to
@@ -3667,10 +3697,6 @@ static bool merges_edges(const gk_solver *s) { return (double)s->ni * s->nj * s-
 // (8, 4) in FP32-bulk within 3%; 256^3 (32, 16) best.  The pair that was the
 // default for every size, (32, 16), had cost 32^3 3.8x and 128x128x8 2.3x.
 // gk_autotune times the candidates on the grid itself.
-//
-// Merged marches share the chip, so they
-// may be longer than a march that has it alone: 2 faces per thread best at
-// 32^3, 4 at 61x43x37, 8 at 48^3, 12 at 128x128x8 and above.
 static void default_shapes(gk_solver *s) {
   const double n = (double)s->ni * s->nj * s->nk;
   if (n >= 1.2e7) {
@@ -3696,7 +3722,7 @@ static void default_shapes(gk_solver *s) {
   s->merge_sweeps = merges_sweeps(s);
   s->merge_edges = merges_edges(s);
   s->merge_asked = 0;
-  s->merge_chunk = n < 5e4 ? 2 : n < 1e5 ? 4 : n < 1.25e5 ? 8 : 12;
+  s->merge_chunk = merge_length(s);
 }
 
 // whether the reconstruction rows of axis a (nf faces) are the same in every
@@ -4616,7 +4642,7 @@ static void plan_step(const gk_solver *s, const Rot &r, std::vector<Launch> &out
       const int wk = a.hi[2] - a.lo[2] + 1;
       const int rem = wk % 64;
       SweepArgs m = a;
-      m.rp = wk <= 32 ? std::min(64 / wk, PACKSPAN / (wk + 7)) : 1;
+      m.rp = pack_rows(wk);
       const bool split = wk >= 64 && rem > 0 && rem < 32;
       if (split) m.hi[2] = a.hi[2] - rem;
       L.kid = SK_SWEEP_K;
