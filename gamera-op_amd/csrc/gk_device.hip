@@ -178,8 +178,9 @@ __device__ __forceinline__ bool halted(const Scal *sc) { return sc && sc->halt; 
 // sweeps' work and traffic, and p_S is zero unless a problem sets it.  While
 // p_S is 0 everywhere and the state is regular (density positive, all of it
 // finite), the step keeps it 0: its flux is 0 and p_S / rho^(gamma-1) is 0.
-// The prologue scans the state (k_scan_entropy) and every cell update reports
-// a p_S that is not 0 or a value that is not finite, from which step on the
+// The prologue scans the state (k_scan_entropy), and every cell update reports
+// a value that is not finite (without the channel a p_S of 0 can only stay 0 or,
+// where the new density is irregular, become NaN), from which step on the
 // kernels carry the channel again.  Two words, as the cell update sets one
 // while other blocks of its launch still read the other; k_begin folds them.
 // 256^3 (sweeps i / j / k, cell update, ghost fill): FP64 0.97 / 0.97 / 1.17,
@@ -2474,7 +2475,7 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
 #pragma unroll
       for (int m = 0; m < 5; m++) st_nt(a.Xn32 + m * g.fs + c, (float)out[m]);
     }
-    if (ent || !(ps == 0.0)) {  // not carried: the buffers hold 0 where nothing is stored
+    if (ent || !(ps == 0.0)) {  // not carried: 0, which the buffers hold, or NaN
       st_nt(a.Xn + 5 * g.fs + c, ps);
       if (a.Xn32) st_nt(a.Xn32 + 5 * g.fs + c, (float)ps);
     }

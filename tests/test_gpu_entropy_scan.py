@@ -126,3 +126,47 @@ def test_scan_costs_the_same_whatever_it_finds():
         assert best[1] < 1.4 * best[0]
     finally:
         S.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("batched", [False, True])
+def test_switched_on_in_mid_run(precision, batched):
+    """A regular state without p_S that turns non-finite in its first step (eight
+    planes of negative pressure: no real sound speed on either side of their
+    faces): from then on the channel is carried.  The twin
+    carries it from the start, for a cell with p_S out of reach: every field
+    of the solver, its NaN among them, is the twin's."""
+    n = (60, 16, 12)
+    P = go.Problem(go.SINUSOID_SPHERE, 85, *n)
+    S, T = go.Solver(P, precision), go.Solver(P, precision)
+    prim, bface = arrays(P)
+    P.close()
+    B = go.Batch() if batched else None
+    try:
+        prim[4][8:16] = -1.0
+        set_state(S, prim, bface)
+        prim[5][48, 10, 9] = 0.25
+        set_state(T, prim, bface)
+        if batched:
+            B.add(S)
+            B.add(T)
+        near = (slice(4, 32), slice(4, 20), slice(4, 16))
+        for step in range(3):
+            if batched:
+                with pytest.raises(go.GkNonFinite):
+                    B.step(1)
+            else:
+                for s in (S, T):
+                    with pytest.raises(go.GkNonFinite):
+                        s.step(1)
+            (ps, bs), (pt, bt) = S.state(), T.state()
+            for x, y in zip(ps[:5] + bs, pt[:5] + bt):
+                assert np.array_equal(x, y, equal_nan=True), step
+            assert np.array_equal(ps[5][near], pt[5][near], equal_nan=True), step
+            assert np.isnan(ps[5][near]).any() and (pt[5][44:52] > 0.0).any()
+    finally:
+        if batched:
+            B.close()
+        S.close()
+        T.close()
