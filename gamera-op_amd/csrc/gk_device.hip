@@ -421,13 +421,17 @@ __device__ __forceinline__ void utab(const Geo &g, int f, R T[GK_RECW_STRIDE]) {
 // with the geometry terms c1, c2 precomputed per face.  |s0 + s1| is 2, 1, 0
 // for equal signs, f0 = f-1, opposite signs, so its product is exact inside a
 // fused multiply-add.  In FP64 the halves are folded too (D = 2 df0c, half the
-// factor), which changes no rounding above 1e-307.  s1 multiplies a number
+// factor), which changes no rounding above 1e-307; below, where halving a
+// number rounds, a state may be a few units of 2^-1074 off the reference's (as it
+// halves, the steps take 0.7 to 1.1 % longer: 256^3 5.83 -> 5.88 ms, 96x72x60 0.295
+// -> 0.298).  s1 multiplies a number
 // that is 0 where s1 is 0 (f0 = f+1 clamps f to f0), so it is a copied sign
 // bit; the other state of the face has the opposite s1.  The signs are read
 // off the high words instead of being formed as -1, 0, 1 (two compares and a
-// select or two each).  The sweeps and edge fields are bound by vector issue (72-92 % busy
-// in the sweeps), and this is 22 vector instructions per state in FP64
-// against 33: 256^3 FP64 i / j / k sweeps 1.06 / 1.04 / 1.22 -> 0.97 / 0.97 /
+// select or two each).  Vector issue is the largest single term of the sweeps and
+// edge fields (VALU 71 / 72 / 51 % busy in the FP64 i / j / k sweeps, 77 / 86 / 69 % in
+// FP32-bulk, 46 to 65 % in the FP64 edge fields), and this is 22 vector instructions
+// per state in FP64 against 33: 256^3 FP64 i / j / k sweeps 1.06 / 1.04 / 1.22 -> 0.97 / 0.97 /
 // 1.17 ms, E_i / E_j / E_k 0.351 / 0.387 / 0.520 -> 0.331 / 0.372 / 0.507 ms,
 // FP32-bulk sweeps 0.46 -> 0.44 ms (there memory binds next).
 __device__ __forceinline__ double limit_q(double d0, double d1) {
