@@ -18,8 +18,9 @@
 //                positivity floors, Boris-corrected momentum; fused CFL min /
 //                |div B| max / NaN reduction for the next step
 //   k_ghost      periodic / symmetric ghost fill of the new state (replaces
-//                the MPI halo exchange and the boundary-condition library)
-//   k_mags       cell-centred B of the new state over the ghosted box
+//                the MPI halo exchange and the boundary-condition library), with
+//                the cell-centred B of the ghost cells (k_cell stores the
+//                active cells'; k_mags forms it over the whole box at set-up)
 //
 // Arithmetic: the FP64 path keeps the reference's floating-point operation
 // order and is built without FMA contraction.  The PDM limiter branches on
@@ -429,8 +430,8 @@ __device__ __forceinline__ void utab(const Geo &g, int f, R T[GK_RECW_STRIDE]) {
 // bit; the other state of the face has the opposite s1.  The signs are read
 // off the high words instead of being formed as -1, 0, 1 (two compares and a
 // select or two each).  Vector issue is the largest single term of the sweeps and
-// edge fields (VALU 71 / 72 / 51 % busy in the FP64 i / j / k sweeps, 77 / 86 / 69 % in
-// FP32-bulk, 46 to 65 % in the FP64 edge fields), and this is 22 vector instructions
+// edge fields (VALU 70 / 72 / 49 % busy in the FP64 i / j / k sweeps, 75 / 84 / 66 % in
+// FP32-bulk, 45 to 63 % in the FP64 edge fields), and this is 22 vector instructions
 // per state in FP64 against 33: 256^3 FP64 i / j / k sweeps 1.06 / 1.04 / 1.22 -> 0.97 / 0.97 /
 // 1.17 ms, E_i / E_j / E_k 0.351 / 0.387 / 0.520 -> 0.331 / 0.372 / 0.507 ms,
 // FP32-bulk sweeps 0.46 -> 0.44 ms (there memory binds next).
@@ -2090,9 +2091,10 @@ __device__ __forceinline__ void k_ct_body(const CtArgs &a, const int bx, const i
 
 // The same update by threads that walk CT_CHUNK points along i (FP64 grids from
 // CT_WALK cells): E_j and E_k at i + 1 are the next point's, and the row and
-// column factors are read once, 12 loads a point instead of 27.  The plain form
-// is bound by its load instructions (address unit 83 % busy at 3.7 of 6.2
-// TB/s): 256^3 0.369 -> 0.329 ms, sphere 128x128x256 0.098 -> 0.088, 128^3 0.052
+// column factors are read once, 15 loads a point instead of 27 (counted over all
+// waves: 62 for four points, 24 for one in FP32-bulk).  Both forms are bound by their
+// load instructions (address unit 83 % busy in the plain one at 3.7 of 6.2 TB/s, 79 %
+// in this one at 4.3): 256^3 0.369 -> 0.329 ms, sphere 128x128x256 0.098 -> 0.088, 128^3 0.052
 // -> 0.050.  Below that the launch
 // is too short to fill the chip with a quarter of the threads (96x72x60 0.0175 ->
 // 0.0192 ms, 32^3 0.007 -> 0.011), and in FP32-bulk, where the stores weigh more,
@@ -2270,8 +2272,8 @@ __device__ __forceinline__ void globalize(CellArgs &a) {
 // kind: the terms cost a Cartesian grid 62 registers in FP64 (193 -> 131, a
 // third wave per SIMD) and 34 in FP32-bulk (162 -> 128, a fourth), and a
 // spherical grid, where they were read behind a branch on a.spherical, a second
-// wait for memory.  Bound by its load instructions (90 a cell in FP64, address
-// unit 85 % busy) at 4.6 and 4.8 of 6.2 TB/s: 256^3 1.46 -> 1.32 ms FP64 and
+// wait for memory.  Bound by its load instructions (82 a cell, beside 8 stores in
+// FP64 and 14 in FP32-bulk; address unit 85 % busy) at 4.7 and 4.9 of 6.2 TB/s: 256^3 1.46 -> 1.32 ms FP64 and
 // 0.93 -> 0.89 ms FP32-bulk; shell 192x96x192 FP32-bulk 0.343 ->
 // 0.252 ms, sphere 128x128x256 FP64 0.445 -> 0.434 ms.  One wave more
 // asked for spills: 1.35, 1.74 ms at 256^3.
@@ -2483,7 +2485,7 @@ __device__ __forceinline__ void k_cell_body(const CellArgs &a, const int bx, con
       st_nt(a.Xn + 5 * g.fs + c, ps);
       if (a.Xn32) st_nt(a.Xn32 + 5 * g.fs + c, (float)ps);
     }
-    // cell-centred B at n+1 (the ghost cells' is formed after the ghost fill)
+    // cell-centred B at n+1 (the ghost fill forms the ghost cells')
 #pragma unroll
     for (int m = 0; m < 3; m++) {
       if (a.Mn) st_nt(a.Mn + m * g.fs + c, bnew[m]);
